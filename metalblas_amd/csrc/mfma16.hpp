@@ -29,6 +29,7 @@
 #pragma once
 
 #include "launch.hpp"
+#include "tile_order.hpp"
 
 namespace mb {
 namespace m16 {
@@ -375,23 +376,6 @@ template <int ROWS, int NW, bool KC, int ES = 2, int MS = 32> struct Tile16 {
     }
 };
 
-__device__ __forceinline__ void tile_coords16(int pid, int tiles_m, int tiles_n, int swz, int &tm, int &tn) {
-    const int n = tiles_m * tiles_n;
-    if (n >= 16) {
-        const int xcd = pid & 7, idx = pid >> 3;
-        const int base = n >> 3, rem = n & 7;
-        pid = xcd * base + min(xcd, rem) + idx;
-    }
-    const int G = 1 << swz;
-    const int width = G * tiles_n;
-    const int grp = pid / width;
-    const int first_m = grp * G;
-    const int gsz = min(tiles_m - first_m, G);
-    const int in = pid - grp * width;
-    tm = first_m + in % gsz;
-    tn = in / gsz;
-}
-
 // Store a wave's accumulators: acc[i][j] holds the MS x MS block at rows mw + MS j, columns
 // nw + MS i; lane l owns row (l % MS) and columns 8 (r / 4) + 4 (l / MS) + r % 4 of register r
 // (MS = 32: 16 registers; MS = 16: 4).
@@ -685,10 +669,9 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm16(GemmArgs g) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave % WM, wn = wave / WM;
     const int tiles_m = cdiv(g.M, BM), tiles_n = cdiv(g.N, BN);
-    int tm, tn;
-    tile_coords16(blockIdx.x, tiles_m, tiles_n, g.swz, tm, tn);
+    int tm, tn, ks, bz0;
+    work_coords(tiles_m, tiles_n, g.swz, tm, tn, ks, bz0);
     const int m0 = tm * BM, n0 = tn * BN;
-    const int ks = blockIdx.y;
     const int kbeg = ks * g.k_chunk;
     const int kend = min(g.K, kbeg + g.k_chunk);
     const int klen = kend - kbeg;
@@ -779,7 +762,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm16(GemmArgs g) {
                 for (int j = 0; j < TM; ++j) mma16<T>(acc[i][j], fb[slot][i], fa[slot][j]);
         };
         zero_acc();
-        int e = blockIdx.z, kt = 0, buf = 0;
+        int e = bz0, kt = 0, buf = 0;
         load_es(e, 0, 0);
         while (true) {
             vm_wait_all();     // this wave's loads of stage (e, kt), and earlier stores
@@ -816,7 +799,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm16(GemmArgs g) {
         return;
     }
 
-    for (int bz = blockIdx.z; bz < g.batch; bz += gridDim.z) {
+    for (int bz = bz0; bz < g.batch; bz += gridDim.z) {
         // resource bases: element (row0, kbeg) of each operand tile
         const T *Ab = (const T *)g.a + bz * g.a_bs + (A_KC ? (int64_t)m0 * lda + kbeg : (int64_t)kbeg * lda + m0);
         const T *Bb = (const T *)g.b + bz * g.b_bs + (B_KC ? (int64_t)n0 * ldb + kbeg : (int64_t)kbeg * ldb + n0);
@@ -979,15 +962,14 @@ __global__ __launch_bounds__(64 * WM * WN) void k_thin16(GemmArgs g) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave % WM, wn = wave / WM;
     const int tiles_m = cdiv(g.M, BM), tiles_n = cdiv(g.N, BN);
-    int tm, tn, ks;
+    int tm, tn, ks, bz0 = blockIdx.z;
     if constexpr (XMAP) {
         int tile;
         slice_coords(blockIdx.x, gridDim.x, tiles_m * tiles_n, tile, ks);
         tm = tile % tiles_m;
         tn = tile / tiles_m;
     } else {
-        tile_coords16(blockIdx.x, tiles_m, tiles_n, g.swz, tm, tn);
-        ks = blockIdx.y;
+        work_coords(tiles_m, tiles_n, g.swz, tm, tn, ks, bz0);
     }
     const int m0 = tm * BM, n0 = tn * BN;
     const int kbeg = ks * g.k_chunk;
@@ -1012,7 +994,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_thin16(GemmArgs g) {
 #pragma unroll
     for (int j = 0; j < (B_KC ? 1 : TN); ++j) fbb[j] = TB::frag_base(wn * WTN, lane, j);
 
-    for (int bz = blockIdx.z; bz < g.batch; bz += gridDim.z) {
+    for (int bz = bz0; bz < g.batch; bz += gridDim.z) {
         const T *Ab = (const T *)g.a + bz * g.a_bs + (A_KC ? (int64_t)m0 * lda + kbeg : (int64_t)kbeg * lda + m0);
         const T *Bb = (const T *)g.b + bz * g.b_bs + (B_KC ? (int64_t)n0 * ldb + kbeg : (int64_t)kbeg * ldb + n0);
         const i32x4 ra = make_rsrc(Ab), rb = make_rsrc(Bb);
@@ -1155,10 +1137,9 @@ __global__ __launch_bounds__(512) void k_gemm16pp(GemmArgs g) {
     const int group = wave >> 2;
     const int wm = wave % WM, wn = wave / WM;
     const int tiles_m = cdiv(g.M, BM), tiles_n = cdiv(g.N, BN);
-    int tm, tn;
-    tile_coords16(blockIdx.x, tiles_m, tiles_n, g.swz, tm, tn);
+    int tm, tn, ks, bz0;
+    work_coords(tiles_m, tiles_n, g.swz, tm, tn, ks, bz0);
     const int m0 = tm * BM, n0 = tn * BN;
-    const int ks = blockIdx.y;
     const int kbeg = ks * g.k_chunk;
     const int kend = min(g.K, kbeg + g.k_chunk);
     const int klen = kend - kbeg;
@@ -1186,7 +1167,7 @@ __global__ __launch_bounds__(512) void k_gemm16pp(GemmArgs g) {
     for (int j = 0; j < (B_KC ? 1 : TN); ++j)
         fbb[j] = MS == 16 ? TB::frag_base16(wn * WTN, lane, j) : TB::frag_base(wn * WTN, lane, j);
 
-    for (int bz = blockIdx.z; bz < g.batch; bz += gridDim.z) {
+    for (int bz = bz0; bz < g.batch; bz += gridDim.z) {
         const T *Ab = (const T *)g.a + bz * g.a_bs + (A_KC ? (int64_t)m0 * lda + kbeg : (int64_t)kbeg * lda + m0);
         const T *Bb = (const T *)g.b + bz * g.b_bs + (B_KC ? (int64_t)n0 * ldb + kbeg : (int64_t)kbeg * ldb + n0);
         const i32x4 ra = make_rsrc(Ab), rb = make_rsrc(Bb);

@@ -29,6 +29,7 @@
 #pragma once
 
 #include "launch.hpp"
+#include "tile_order.hpp"
 
 namespace mb {
 
@@ -209,25 +210,6 @@ template <class T, int ROWS, int NT, bool KC> struct TileLoader {
     }
 };
 
-// Logical tile index from the hardware workgroup id: XCD-contiguous ranges, then groups of
-// 2^swz tile rows walked column by column.
-__device__ __forceinline__ void tile_coords(int pid, int tiles_m, int tiles_n, int swz, int &tm, int &tn) {
-    const int n = tiles_m * tiles_n;
-    if (n >= 16) {
-        const int xcd = pid & 7, idx = pid >> 3;
-        const int base = n >> 3, rem = n & 7;
-        pid = xcd * base + min(xcd, rem) + idx;
-    }
-    const int G = 1 << swz;
-    const int width = G * tiles_n;
-    const int grp = pid / width;
-    const int first_m = grp * G;
-    const int gsz = min(tiles_m - first_m, G);
-    const int in = pid - grp * width;
-    tm = first_m + in % gsz;
-    tn = in / gsz;
-}
-
 template <class T, int BM, int BN, int WM, int WN, bool A_KC, bool B_KC>
 __global__ __launch_bounds__(64 * WM * WN) void k_gemm_mfma(GemmArgs g) {
     using P = Pol<T>;
@@ -245,10 +227,9 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_mfma(GemmArgs g) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave % WM, wn = wave / WM;
     const int tiles_m = cdiv(g.M, BM), tiles_n = cdiv(g.N, BN);
-    int tm, tn;
-    tile_coords(blockIdx.x, tiles_m, tiles_n, g.swz, tm, tn);
+    int tm, tn, ks, bz0;
+    work_coords(tiles_m, tiles_n, g.swz, tm, tn, ks, bz0);
     const int m0 = tm * BM, n0 = tn * BN;
-    const int ks = blockIdx.y;
     const int kbeg = ks * g.k_chunk;
     const int kend = min(g.K, kbeg + g.k_chunk);
     const int nk = cdiv(kend - kbeg, BK);
@@ -257,7 +238,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_mfma(GemmArgs g) {
     const int64_t lda = A_KC ? g.a_rs : g.a_cs;
     const int64_t ldb = B_KC ? g.b_cs : g.b_rs;
 
-    for (int bz = blockIdx.z; bz < g.batch; bz += gridDim.z) {
+    for (int bz = bz0; bz < g.batch; bz += gridDim.z) {
         const T *Ab = (const T *)g.a + bz * g.a_bs;
         const T *Bb = (const T *)g.b + bz * g.b_bs;
 
