@@ -520,7 +520,7 @@ def main(argv=None):
             "frac": round(tf / PEAK["bf16"], 4),
             "traffic": TRAFFIC["bf16_gemm_8192"] if n == 8192 else None,
             "kernel": f"matrix-core GEMM tile {plan['tile'][0]}x{plan['tile'][1]} "
-                      f"schedule {'ping-pong' if plan['tile'][5] == 2 else 'interleaved'}",
+                      f"schedule {({2: 'ping-pong', 4: 'K ping-pong'}).get(plan['tile'][5], 'interleaved')}",
             "algorithmic_per_launch": f"2*{n}^3 = {w.flops:.4e} flop",
             "avg_launch_ms": round(ms, 4),
         }

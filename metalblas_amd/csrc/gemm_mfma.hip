@@ -17,8 +17,10 @@ hipError_t launch_bf16_kwhole(const MfmaTile &, bool, bool, const GemmArgs &, di
 hipError_t launch_bf16_ktail(const MfmaTile &, bool, bool, const GemmArgs &, dim3, hipStream_t);
 hipError_t launch_f16_kwhole(const MfmaTile &, bool, bool, const GemmArgs &, dim3, hipStream_t);
 hipError_t launch_f16_ktail(const MfmaTile &, bool, bool, const GemmArgs &, dim3, hipStream_t);
-hipError_t launch_bf16_pp(bool ktail, int bn, bool, bool, const GemmArgs &, dim3, hipStream_t);
-hipError_t launch_f16_pp(bool ktail, int bn, bool, bool, const GemmArgs &, dim3, hipStream_t);
+hipError_t launch_bf16_pp(bool ktail, bool, bool, const GemmArgs &, dim3, hipStream_t);
+hipError_t launch_f16_pp(bool ktail, bool, bool, const GemmArgs &, dim3, hipStream_t);
+hipError_t launch_bf16_kpp(bool ktail, int bm, bool, bool, const GemmArgs &, dim3, hipStream_t);
+hipError_t launch_f16_kpp(bool ktail, int bm, bool, bool, const GemmArgs &, dim3, hipStream_t);
 hipError_t launch_i8_kwhole(const MfmaTile &, bool, bool, const GemmArgs &, dim3, hipStream_t);
 hipError_t launch_i8_ktail(const MfmaTile &, bool, bool, const GemmArgs &, dim3, hipStream_t);
 hipError_t launch_i8_pp(bool ktail, bool, bool, const GemmArgs &, dim3, hipStream_t);
@@ -37,9 +39,8 @@ constexpr TileEntry kTiles[] = {
     {128, 64, 2, 2, 0},  {64, 128, 2, 2, 0},  {64, 64, 2, 2, 0},   {32, 32, 1, 1, 0},
 };
 // LDS-direct family (mfma16.hpp): bf16 / fp16 / int8 / uint8; sched 1 = the ping-pong kernel
-// (256 x 128 ping-pong: bf16 / fp16 only)
 constexpr TileEntry kTiles16[] = {
-    {256, 256, 2, 4, 1}, {256, 128, 2, 4, 1}, {256, 256, 2, 2, 0}, {256, 256, 2, 4, 0}, {256, 128, 2, 2, 0}, {128, 256, 2, 2, 0},
+    {256, 256, 2, 4, 1}, {256, 256, 2, 2, 0}, {256, 256, 2, 4, 0}, {256, 128, 2, 2, 0}, {128, 256, 2, 2, 0},
     {128, 128, 2, 2, 0}, {128, 64, 2, 2, 0},  {64, 128, 2, 2, 0},  {64, 64, 2, 2, 0},  {32, 32, 1, 1, 0},
     // thin tiles for products with a few vectors (bf16 / fp16): k_thin_dot 64 x 16 and
     // k_thin_dot4 4 x 16 (A and B K-contiguous), k_thin16 32 x 256 and 32 x 128 (A
@@ -48,6 +49,9 @@ constexpr TileEntry kTiles16[] = {
     {64, 16, 4, 1, 0},   {32, 256, 1, 4, 0},  {32, 128, 1, 4, 0}, {4, 16, 1, 1, 0},  {4, 8, 16, 1, 0},
     // the deep-K schedule of the 64 x 64 tile (bf16 / fp16): few output tiles, many K slices
     {64, 64, 2, 2, 2},
+    // K ping-pong (mfma_kpp.hpp): two groups of four waves share the K of a 128 x 128 or
+    // 256 x 128 tile (bf16 / fp16)
+    {128, 128, 2, 4, 3}, {256, 128, 2, 4, 3},
 };
 
 // dtypes of the LDS-direct family
@@ -78,8 +82,7 @@ bool mfma_supported_dtype(int dt) { return dt == BF16 || dt == F16 || dt == F32 
 int mfma_k_align(int dt) { return 16 / dtype_size(dt); }
 
 bool mfma_tile_compiled(int dt, const MfmaTile &t) {
-    if ((dt == I8 || dt == U8) && t.sched == 1 && t.bn != 256) return false;   // 8-bit ping-pong: 256 x 256 only
-    if (t.sched == 2 && dt != BF16 && dt != F16) return false;                  // deep-K: 16-bit floats only
+    if (t.sched >= 2 && dt != BF16 && dt != F16) return false;   // deep-K, K ping-pong: 16-bit floats only
     if (is16(dt)) return in_table(kTiles16, sizeof(kTiles16) / sizeof(kTiles16[0]), t);
     return in_table(kTiles, sizeof(kTiles) / sizeof(kTiles[0]), t);
 }
@@ -90,7 +93,7 @@ int mfma_list_tiles(int dt, MfmaTile *out, int cap) {
     int n = 0;
     for (int i = 0; i < cnt; ++i) {
         const MfmaTile t{tb[i].bm, tb[i].bn, tb[i].wm, tb[i].wn, tb[i].sched};
-        if (!mfma_tile_compiled(dt, t)) continue;   // e.g. the 8-bit ping-pong exists at 256 x 256 only
+        if (!mfma_tile_compiled(dt, t)) continue;   // e.g. K ping-pong: 16-bit floats only
         if (n < cap) out[n] = t;
         ++n;
     }
@@ -115,10 +118,14 @@ hipError_t launch_mfma(int dt, const MfmaTile &t, bool a_kc, bool b_kc, const Ge
                 if (shape) *shape = {g1, dim3(256)};
                 return m16::launch_deepk(dt, !whole, a_kc, b_kc, g, g1, st);
             }
+            if (t.sched == 3) {
+                if (dt == BF16) return m16::launch_bf16_kpp(!whole, t.bm, a_kc, b_kc, g, grid, st);
+                if (dt == F16) return m16::launch_f16_kpp(!whole, t.bm, a_kc, b_kc, g, grid, st);
+                return hipErrorInvalidValue;
+            }
             if (t.sched == 1) {
-                if (dt == BF16) return m16::launch_bf16_pp(!whole, t.bn, a_kc, b_kc, g, grid, st);
-                if (dt == F16) return m16::launch_f16_pp(!whole, t.bn, a_kc, b_kc, g, grid, st);
-                if (t.bn != 256) return hipErrorInvalidValue;
+                if (dt == BF16) return m16::launch_bf16_pp(!whole, a_kc, b_kc, g, grid, st);
+                if (dt == F16) return m16::launch_f16_pp(!whole, a_kc, b_kc, g, grid, st);
                 return m16::launch_i8_pp(!whole, a_kc, b_kc, g, grid, st);   // int8 and uint8
             }
             if (dt == BF16)

@@ -490,34 +490,39 @@ void plan_mfma(const Prob &p, Plan &pl, bool a_kc, bool b_kc, bool thin_ok = fal
         // per CU x BM*BN*K_slice / eff, plus the split-K reduction (partial planes written and
         // read at ~5 TB/s, and a launch).  occ = workgroups per CU (LDS/VGPR limited); eff =
         // relative per-CU throughput, measured on MI355X (bf16 8192^3, 4096^3, 2048^2 x 4096,
-        // 1024^2 x 8192, 4096 x 1024 x 4096; 256 x 128 against 128 x 128 on 2048 x 4096 x 2048
-        // and 8192 x 1024 x 1024, where 128 x 128 is 4-6 % faster).
+        // 1024^2 x 8192, 4096 x 1024 x 4096; the K ping-pong tiles on 2048 x 2048 x 4096, 2560^3,
+        // 3072^3 and 2048 x 4096 x 2048).
         struct Cand {
             MfmaTile t;
             int occ;
             double eff;
         };
         static const Cand cands[] = {
-            {{256, 256, 2, 4, 1}, 1, 1.00}, {{256, 128, 2, 4, 1}, 1, 0.90}, {{256, 256, 2, 2}, 1, 0.85},
+            {{256, 256, 2, 4, 1}, 1, 1.00}, {{256, 128, 2, 4, 3}, 1, 0.95}, {{256, 256, 2, 2}, 1, 0.85},
             {{256, 128, 2, 2}, 1, 0.66},
-            {{128, 256, 2, 2}, 1, 0.66}, {{128, 128, 2, 2}, 1, 0.70}, {{128, 64, 2, 2}, 2, 0.65},
+            {{128, 256, 2, 2}, 1, 0.66}, {{128, 128, 2, 4, 3}, 1, 0.95}, {{128, 128, 2, 2}, 1, 0.70}, {{128, 64, 2, 2}, 2, 0.65},
             {{64, 128, 2, 2}, 2, 0.60},  {{64, 64, 2, 2}, 3, 0.40},
         };
         const int bk = 128 / dtype_size(p.dt);
         double best = 1e300;
         t = {64, 64, 2, 2};
         for (const auto &c : cands) {
-            if (!mfma_tile_compiled(p.dt, c.t)) continue;   // the 256 x 128 ping-pong is 16-bit float only
+            if (!mfma_tile_compiled(p.dt, c.t)) continue;   // 256 x 128 and K ping-pong: 16-bit floats only
             const int64_t tiles = ((p.M + c.t.bm - 1) / c.t.bm) * ((p.N + c.t.bn - 1) / c.t.bn) * p.batch;
-            const int64_t s = auto_splits(p, tiles, bk);
-            // the 256 x 128 ping-pong tile only unsplit: split over K it measured slower than
-            // the 128 x 128 tile (2056 x 2048 x 4096: 80.8 us at 4 slices against 51.4)
-            if (c.t.sched == 1 && c.t.bn == 128 && s > 1) continue;
+            // the K ping-pong tiles run unsplit unless asked: its waves already share K (1536 x
+            // 1536 x 4096, 144 tiles: 33 us, 50 us over 4 slices, 39 us on the best other tile)
+            const bool kpp = c.t.sched == 3;
+            const int64_t s = kpp && p.split_req == 0 ? 1 : auto_splits(p, tiles, bk);
             const int64_t wgs = tiles * s, slots = (int64_t)cus * c.occ;
             const int64_t rounds = (wgs + slots - 1) / slots;
             const int64_t per_cu = std::min<int64_t>(c.occ, (wgs + cus - 1) / cus);
             const int64_t kc = (p.K + s - 1) / s;
             double cost = (double)rounds * per_cu * c.t.bm * c.t.bn * (double)kc / c.eff;
+            // K ping-pong: its ring fills the CU's LDS, so nothing overlaps the start and the end of
+            // a tile with the next one's (~4 us a round; 8192 x 1024 x 1024: 24.5 us in two rounds of
+            // 128 x 128 against 22.2 in one of 256 x 128; one round of 2048 x 2048 x 4096: 32.7 us
+            // against 41.5 on the interleaved tile)
+            if (kpp) cost += (double)(rounds - 1) * 9e6;
             if (s > 1) cost += (double)s * p.M * p.N * p.batch * 3.84 + 7.2e6;
             if (cost < best * 0.999) {
                 best = cost;
@@ -571,7 +576,7 @@ void plan_mfma(const Prob &p, Plan &pl, bool a_kc, bool b_kc, bool thin_ok = fal
     const int es = dtype_size(p.dt);
     const int BK = 8 * (16 / es);
     const int64_t tiles = ((p.M + t.bm - 1) / t.bm) * ((p.N + t.bn - 1) / t.bn) * p.batch;
-    int64_t splits = auto_splits(p, tiles, BK);
+    int64_t splits = t.sched == 3 && p.split_req == 0 ? 1 : auto_splits(p, tiles, BK);
     if (deepk) {
         splits = std::min<int64_t>(cus / tiles, p.K / 1024);
     } else if (thin) {
