@@ -121,8 +121,9 @@ __global__ __launch_bounds__(256) void k_fill(GemmArgs g) {
 // planes sub, sub+TPO, ... (four independent partial sums), and the TPO partials are added
 // in a fixed order through LDS, so the result is deterministic.  Threads with the same sub
 // read consecutive outputs (coalesced).
-template <class T, int TPO>
+template <class T, int TPO, bool GUARD>
 __global__ __launch_bounds__(256) void k_splitk_reduce(GemmArgs g) {
+    if (GUARD && *g.guard != g.guard_val) return;
     using A = typename Tr<T>::acc;
     constexpr int OPB = 256 / TPO;   // outputs per block iteration
     __shared__ A part[TPO][OPB];
@@ -160,8 +161,9 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(GemmArgs g) {
 
 // The same reduction for fp32 partials with N % 4 == 0: each thread sums 4 consecutive outputs
 // of one row with 16-byte loads (same summation order per output as k_splitk_reduce).
-template <class T, int TPO>
+template <class T, int TPO, bool GUARD>
 __global__ __launch_bounds__(256) void k_splitk_reduce4(GemmArgs g) {
+    if (GUARD && *g.guard != g.guard_val) return;
     constexpr int OPB = 256 / TPO;   // 4-output groups per block iteration
     __shared__ float4 part[TPO][OPB];
     const int64_t plane = (int64_t)g.batch * g.M * g.N;
@@ -205,8 +207,9 @@ __global__ __launch_bounds__(256) void k_splitk_reduce4(GemmArgs g) {
 // Operand copy (PackArgs): each thread writes 4 consecutive elements along the destination's
 // contiguous dimension (coalesced stores); source reads follow the source strides.  The grid
 // is x: inner chunks, y: outer index (grid-stride), z: batch (grid-stride).
-template <class E>
+template <class E, bool GUARD = false>
 __global__ __launch_bounds__(256) void k_pack(PackArgs a) {
+    if (GUARD && *a.guard != a.guard_val) return;
     const int64_t inner_n = a.contig_cols ? a.cols_p : a.rows_p;
     const int64_t outer_n = a.contig_cols ? a.rows_p : a.cols_p;
     const int64_t i0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
@@ -294,8 +297,9 @@ __global__ __launch_bounds__(256) void k_pack16_rows2(PackArgs a0, PackArgs a1, 
 
 // Bhat expansion (CplxExpandArgs): thread per (n, k pair-block) writes the two K-adjacent
 // pairs of Bhat's columns 2n and 2n + 1; the padding k' in [2K, ld) is zero-filled.
-template <class R>
+template <class R, bool GUARD = false>
 __global__ __launch_bounds__(256) void k_cplx_expand(CplxExpandArgs a) {
+    if (GUARD && *a.guard != a.guard_val) return;
     const int64_t kp = a.ld / 2;   // complex k positions per Bhat column, padding included
     const int64_t total = (int64_t)a.N * kp;
     const R sa = a.neg_a ? R(-1.f) : R(1.f), sb = a.neg_b ? R(-1.f) : R(1.f);
@@ -330,10 +334,13 @@ inline int elementwise_blocks(int64_t total) {
 hipError_t launch_cplx_expand(const CplxExpandArgs &a, hipStream_t st) {
     const int64_t total = (int64_t)a.N * (a.ld / 2);
     int64_t blocks = (total + 255) / 256;
-    if (blocks > 16384) blocks = 16384;
+    const int64_t cap = a.guard ? 2048 : 16384;   // guarded: as a rule nothing but the guard is read
+    if (blocks > cap) blocks = cap;
     dim3 grid((unsigned)(blocks < 1 ? 1 : blocks), (unsigned)(a.batch < 65535 ? a.batch : 65535));
     if (a.half)
         hipLaunchKernelGGL(k_cplx_expand<f16_t>, grid, dim3(256), 0, st, a);
+    else if (a.guard)
+        hipLaunchKernelGGL((k_cplx_expand<float, true>), grid, dim3(256), 0, st, a);
     else
         hipLaunchKernelGGL(k_cplx_expand<float>, grid, dim3(256), 0, st, a);
     return hipGetLastError();
@@ -371,8 +378,14 @@ hipError_t launch_pack(const PackArgs &a, hipStream_t st) {
     switch (a.es) {
         case 1: hipLaunchKernelGGL(k_pack<uint8_t>, grid, dim3(256), 0, st, a); break;
         case 2: hipLaunchKernelGGL(k_pack<uint16_t>, grid, dim3(256), 0, st, a); break;
-        case 4: hipLaunchKernelGGL(k_pack<uint32_t>, grid, dim3(256), 0, st, a); break;
-        case 8: hipLaunchKernelGGL(k_pack<uint64_t>, grid, dim3(256), 0, st, a); break;
+        case 4:
+            if (a.guard) hipLaunchKernelGGL((k_pack<uint32_t, true>), grid, dim3(256), 0, st, a);
+            else hipLaunchKernelGGL(k_pack<uint32_t>, grid, dim3(256), 0, st, a);
+            break;
+        case 8:
+            if (a.guard) hipLaunchKernelGGL((k_pack<uint64_t, true>), grid, dim3(256), 0, st, a);
+            else hipLaunchKernelGGL(k_pack<uint64_t>, grid, dim3(256), 0, st, a);
+            break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -399,36 +412,41 @@ hipError_t launch_fill(int dt, const GemmArgs &g, hipStream_t st) {
     });
 }
 
-hipError_t launch_splitk_reduce(int dt, const GemmArgs &g, hipStream_t st) {
+template <class T, bool GUARD> static hipError_t launch_reduce_t(const GemmArgs &g, hipStream_t st) {
     const int64_t plane = (int64_t)g.batch * g.M * g.N;
     // threads per output: enough that a block covers ~8 planes per thread
     const int tpo = g.splits >= 128 ? 16 : g.splits >= 64 ? 8 : (g.splits >= 16 ? 4 : (g.splits >= 4 ? 2 : 1));
     const int64_t opb = 256 / tpo;
-    int64_t blocks = (plane + opb - 1) / opb;
+    const bool four = std::is_same_v<typename Tr<T>::acc, float> && g.N % 4 == 0 && ((uintptr_t)g.ws & 15) == 0;
+    int64_t blocks = ((four ? plane / 4 : plane) + opb - 1) / opb;
     if (blocks > 8192) blocks = 8192;
-    return with_dtype(dt, [&]<class T>() {
+    auto go = [&]<int TPO>() {
         if constexpr (std::is_same_v<typename Tr<T>::acc, float>) {
-            if (g.N % 4 == 0 && ((uintptr_t)g.ws & 15) == 0) {
-                int64_t b4 = (plane / 4 + opb - 1) / opb;
-                if (b4 > 8192) b4 = 8192;
-                switch (tpo) {
-                    case 16: hipLaunchKernelGGL((k_splitk_reduce4<T, 16>), dim3(b4), dim3(256), 0, st, g); break;
-                    case 8: hipLaunchKernelGGL((k_splitk_reduce4<T, 8>), dim3(b4), dim3(256), 0, st, g); break;
-                    case 4: hipLaunchKernelGGL((k_splitk_reduce4<T, 4>), dim3(b4), dim3(256), 0, st, g); break;
-                    case 2: hipLaunchKernelGGL((k_splitk_reduce4<T, 2>), dim3(b4), dim3(256), 0, st, g); break;
-                    default: hipLaunchKernelGGL((k_splitk_reduce4<T, 1>), dim3(b4), dim3(256), 0, st, g); break;
-                }
+            if (four) {
+                hipLaunchKernelGGL((k_splitk_reduce4<T, TPO, GUARD>), dim3(blocks), dim3(256), 0, st, g);
                 return hipGetLastError();
             }
         }
-        switch (tpo) {
-            case 16: hipLaunchKernelGGL((k_splitk_reduce<T, 16>), dim3(blocks), dim3(256), 0, st, g); break;
-            case 8: hipLaunchKernelGGL((k_splitk_reduce<T, 8>), dim3(blocks), dim3(256), 0, st, g); break;
-            case 4: hipLaunchKernelGGL((k_splitk_reduce<T, 4>), dim3(blocks), dim3(256), 0, st, g); break;
-            case 2: hipLaunchKernelGGL((k_splitk_reduce<T, 2>), dim3(blocks), dim3(256), 0, st, g); break;
-            default: hipLaunchKernelGGL((k_splitk_reduce<T, 1>), dim3(blocks), dim3(256), 0, st, g); break;
-        }
+        hipLaunchKernelGGL((k_splitk_reduce<T, TPO, GUARD>), dim3(blocks), dim3(256), 0, st, g);
         return hipGetLastError();
+    };
+    switch (tpo) {
+        case 16: return go.template operator()<16>();
+        case 8: return go.template operator()<8>();
+        case 4: return go.template operator()<4>();
+        case 2: return go.template operator()<2>();
+        default: return go.template operator()<1>();
+    }
+}
+
+hipError_t launch_splitk_reduce(int dt, const GemmArgs &g, hipStream_t st) {
+    // only fp32 and complex64 products run behind a guard (a template argument: a test of the
+    // pointer at the head of the kernel cost every reduction 0.3-0.5 us)
+    return with_dtype(dt, [&]<class T>() {
+        if constexpr (std::is_same_v<T, float> || std::is_same_v<T, c64_t>) {
+            if (g.guard) return launch_reduce_t<T, true>(g, st);
+        }
+        return launch_reduce_t<T, false>(g, st);
     });
 }
 

@@ -88,6 +88,8 @@ struct PackArgs {
     int32_t rows, cols, rows_p, cols_p, batch;
     int32_t contig_cols;   // 1: destination contiguous along columns (d_cs == 1), else rows
     int32_t es;            // element bytes: 1, 2, 4 or 8
+    const int32_t *guard;  // as GemmArgs::guard (4- and 8-byte elements)
+    int32_t guard_val;
 };
 
 // Complex product as a real one: C (M x N complex) = A (M x K complex) @ B (K x N complex) is
@@ -104,7 +106,37 @@ struct CplxExpandArgs {
     int32_t K, N, batch;
     int32_t neg_a, neg_b;       // conj(A), conj(B)
     int32_t half;               // 1: complex32 (fp16 parts), 0: complex64 (fp32 parts)
+    const int32_t *guard;       // as GemmArgs::guard
+    int32_t guard_val;
 };
+
+// One operand of an fp32 / complex64 product on the fp16 matrix cores (gemm_split32.hip): row r
+// (M or N index), source k at src[r * rs + k * ks + batch * bs], in elements of the source type.
+// Stored row r holds the real K' = K (complex: 2K, re and im in turn) padded with zeros to Kp, per
+// 32 k 32 hi then 32 lo halves.
+struct SplitOperand {
+    const void *src;
+    int64_t rs, ks, bs;
+    void *dst;             // split planes: row r at dst + r * ld halves
+    int64_t ld, d_bs;
+    uint32_t *part;        // largest magnitudes [batch][slices][part_ld]
+    int32_t *exps;         // exponent that undoes a row's scaling, [batch][R]
+    int32_t R, K, Kp, batch;
+    int32_t k_contig;      // ks == 1 (or no unit stride): read along K, else along the rows
+    int32_t k_slice, slices, part_ld;
+    int32_t cplx;
+    float min_x;           // scaled magnitudes below this (but not 0) raise the flag
+};
+struct SplitExps {
+    const int32_t *ea, *eb;
+    int64_t ea_bs, eb_bs;
+    const int32_t *flag;
+};
+// the row magnitudes of both operands (clears *flag), then their split planes (may raise *flag); an
+// operand with R == 0 is left out
+hipError_t launch_split_absmax(const SplitOperand &a, const SplitOperand &b, int32_t *flag, hipStream_t st);
+hipError_t launch_split32(const SplitOperand &a, const SplitOperand &b, int32_t *flag, hipStream_t st);
+hipError_t launch_gemm_split32(bool cplx, const GemmArgs &g, const SplitExps &x, hipStream_t st);
 
 // gemm_generic.hip
 hipError_t launch_cplx_expand(const CplxExpandArgs &a, hipStream_t st);

@@ -1186,9 +1186,23 @@ constexpr uint64_t kSentSpan = uint64_t(1) << 52;   // one span per operand: a, 
 // spans 4..6: the workspace copies of a packed peel (placed at run time)
 constexpr uint64_t kSentCopy = kSentBase + 4 * kSentSpan;
 
+// An fp32 / complex64 product split over the fp16 matrix cores (gemm_split32.hip).  The workspace
+// holds the flag, then (shared: they run one after another) the split's arrays or the workspace
+// of the fp32 plan behind it.
+struct Split32 {
+    bool on = false, cplx = false;
+    int panels = 1;                           // panels of A rows, split and multiplied in turn
+    SplitOperand a{}, b{};                    // pointers into the workspace set at run time
+    int64_t part[2], exps[2], dst[2];         // workspace byte offsets of their arrays
+    GemmArgs g{};
+    int64_t planes = 0;                       // split-K partial planes
+    int64_t ws_bytes = 0;
+};
+
 struct CallPlan {
     int n = 0;       // launch sequences: 1, or the 2-3 parts of a peeled product
     Plan part[3];
+    Split32 sp;      // on: runs first, the parts are the fp32 plan it may leave the product to
     int ncopy = 0;   // packed peel: operand copies made before the parts
     PackOp copy[3];  // (their .off is the workspace offset; the parts' workspace follows)
     int64_t copy_bytes = 0;
@@ -1292,7 +1306,160 @@ bool plan_packed_peel(const mb_gemm_desc *d, CallPlan &cp, bool sizing) {
     return true;
 }
 
+// ---- fp32 / complex64 on the fp16 matrix cores ---------------------------------------------------
+// Taken under the AUTO backend, without a tile or split request, when the fp32 plan would run on
+// the matrix cores and the product is large enough to repay its three extra launches (the
+// magnitudes, the split, the fp32 kernels that find the flag down).
+constexpr int64_t kSplitFlagBytes = 256;
+// Real multiply-adds below which the fp32 kernels win, and per real operand element: the split
+// moves each element twice more.  Measured on MI355X (us, fp32 kernels -> split): fp32 1280^3 65 ->
+// 51, 1024 x 1024 x 2048 66 -> 50, 2048^3 166 -> 83, 4096^3 1081 -> 470, 512 x 4096 x 1024 54 -> 52;
+// kept: 1024^3 36 (48), 16 x 512^3 49 (55), 128 x 512 x 512 x 64 100 (133); complex64, whose fp32
+// plan expands B: 768^3 75 -> 49, 512 x 1024 x 768 56 -> 48; kept: 512^3 34 (39).
+constexpr double kSplitMinWorkF32 = 2e9, kSplitMinWorkC64 = 1.3e9, kSplitMinPerElem = 400;
+constexpr int64_t kSplitMaxBytes = (int64_t)8 << 30;         // workspace
+// The workspace that the Python layer keeps per stream and mb_gemm_noalloc holds: a product whose
+// fp32 plan fits it keeps fitting it where panels of A rows allow that.
+constexpr int64_t kSplitKeptBytes = kScratchBytes;
+
+// The fp32 plan behind the split in cp.part[0 .. n-1]: one plan, or two halves of the columns when
+// one alone would fill the kept workspace and leave no room for the flag.
+bool plan_split_fallback(const mb_gemm_desc *d, CallPlan &cp) {
+    cp.n = 1;
+    cp.part[0] = Plan();
+    if (make_plan(d, cp.part[0]) != MB_OK || cp.part[0].family != MB_FAMILY_MFMA) return false;
+    const int64_t ws = cp.part[0].ws_bytes;
+    if (ws > kSplitKeptBytes || ws + kSplitFlagBytes <= kSplitKeptBytes || d->N < 256) return true;
+    const int es = dtype_size(d->dtype);
+    const int64_t n1 = d->N / 2 / 64 * 64;
+    auto at = [es](void *ptr, int64_t elems) { return ptr ? (void *)((char *)ptr + elems * es) : ptr; };
+    mb_gemm_desc h[2] = {*d, *d};
+    h[0].N = n1;
+    h[1].N = d->N - n1;
+    h[1].b.ptr = at(d->b.ptr, n1 * d->b.col_stride);
+    h[1].c.ptr = at(d->c.ptr, n1 * d->c.col_stride);
+    h[1].bias.ptr = at(d->bias.ptr, n1 * d->bias.col_stride);
+    for (int i = 0; i < 2; ++i) {
+        cp.part[i] = Plan();
+        if (make_plan(&h[i], cp.part[i]) != MB_OK || cp.part[i].family != MB_FAMILY_MFMA) return false;
+    }
+    cp.n = 2;
+    return true;
+}
+
+bool plan_split32(const mb_gemm_desc *d, CallPlan &cp, bool sizing) {
+    if (d->dtype != MB_DTYPE_F32 && d->dtype != MB_DTYPE_C64) return false;
+    if (d->backend != MB_BACKEND_AUTO || d->tile[0] > 0 || d->tile[1] > 0 || d->split_k != 0) return false;
+    if (!sizing && !d->workspace) return false;
+    Prob p;
+    if (normalise(d, p) != MB_OK || p.batch == 0 || p.M <= 32 || p.N <= 32 || p.K < 32) return false;
+    const bool cplx = p.dt == MB_DTYPE_C64;
+    const double work = (double)p.M * p.N * p.K * p.batch * (cplx ? 4 : 1);
+    if (work < (cplx ? kSplitMinWorkC64 : kSplitMinWorkF32)) return false;
+    const double elems = (double)p.K * (cplx ? 2 : 1) *
+                         ((p.a.bs == 0 ? 1.0 : p.batch) * p.M + (p.b.bs == 0 ? 1.0 : p.batch) * p.N);
+    if (work < kSplitMinPerElem * elems) return false;
+    cp.sp = Split32();
+    Split32 &sp = cp.sp;
+    cp.ncopy = 0;
+    cp.copy_bytes = 0;
+    if (!plan_split_fallback(d, cp)) return false;
+    int64_t fallback_ws = 0;
+    for (int i = 0; i < cp.n; ++i) fallback_ws = std::max<int64_t>(fallback_ws, cp.part[i].ws_bytes);
+    if (p.c.cs != 1 && p.c.rs == 1) transpose(p);
+    const int nc = cplx ? 2 : 1;
+    const int64_t Kr = p.K * nc, Kp = (Kr + 31) / 32 * 32, ld = 2 * Kp, bn = cplx ? 64 : 128;
+    if (Kp >= (int64_t)1 << 21 || p.N > kI32Max / 4 || p.M > kI32Max / 4) return false;   // 31-bit tile offsets
+    const int T = std::min(36, 25 + ilog2_floor(Kr));
+    const float min_x = ldexpf(1.f, 14 - T);
+    for (int which = 0; which < 2; ++which) {
+        const bool is_a = which == 0;
+        const Operand &o = is_a ? p.a : p.b;
+        SplitOperand &s = is_a ? sp.a : sp.b;
+        s.src = o.ptr;
+        s.rs = is_a ? o.rs : o.cs;
+        s.ks = is_a ? o.cs : o.rs;
+        s.bs = o.bs;
+        s.k_contig = s.ks == 1 || s.rs != 1;
+        s.R = s.part_ld = (int)(is_a ? p.M : p.N);
+        s.K = (int)p.K;
+        s.Kp = (int)Kp;
+        s.batch = o.bs == 0 ? 1 : (int)p.batch;
+        s.cplx = cplx;
+        s.min_x = min_x;
+        s.ld = ld;
+        s.d_bs = s.batch == 1 ? 0 : s.R * ld;
+        // K slices of the magnitude pass: enough blocks for the chip, at most 32 partials a row
+        const int64_t unit = s.k_contig ? 1024 : 64;
+        s.k_slice = (int)std::max<int64_t>(unit, ((p.K + 31) / 32 + 63) / 64 * 64);
+        s.slices = (int)((p.K + s.k_slice - 1) / s.k_slice);
+        const int64_t blocks = ((int64_t)s.R + 3) / 4 * std::max<int64_t>(s.slices, (Kp + 63) / 64);
+        if (blocks > kI32Max / 4) return false;
+    }
+    GemmArgs &g = sp.g;
+    fill_gemm_args(p, g);
+    g.K = (int)ld;
+    g.a = g.b = nullptr;
+    g.a_rs = ld; g.a_cs = 1; g.a_bs = sp.a.d_bs;
+    g.b_rs = 1; g.b_cs = ld; g.b_bs = sp.b.d_bs;
+    g.vec_ok = p.c.cs == 1 && p.c.rs % (4 / nc) == 0 && aligned(p.c.ptr, 16) && (p.batch == 1 || p.c.bs % (4 / nc) == 0);
+    const int64_t tiles_m = (p.M + 127) / 128, tiles_n = (p.N + bn - 1) / bn, tiles = tiles_m * tiles_n * p.batch;
+    if (tiles > kI32Max) return false;
+    g.swz = tiles_m >= 8 ? 3 : ilog2_floor(tiles_m);
+    // K slices of at least 8 stages when the tiles leave CUs idle
+    const int64_t stages = Kp / 32;
+    int64_t splits = std::min<int64_t>(std::min<int64_t>(dev_info().cus / tiles, stages / 8), 16);
+    if (splits > 1) {
+        const int64_t per = (stages + splits - 1) / splits;
+        splits = (stages + per - 1) / per;
+        g.k_chunk = (int)(per * 64);
+    }
+    g.splits = (int)std::max<int64_t>(splits, 1);
+    if (g.splits == 1) g.k_chunk = g.K;
+    // Workspace.  Panels of A rows (the next is split after the last one's product) while the whole
+    // exceeds the kept workspace and a panel's tiles still fill the CUs; not with a bias, which may
+    // be C itself: a later panel can still raise the flag, and the fp32 plan then reads the bias.
+    auto lay_out = [&](int panels) {
+        int64_t off = kSplitFlagBytes;
+        auto take = [&off](int64_t bytes) {
+            const int64_t at = off;
+            off += (bytes + 255) / 256 * 256;
+            return at;
+        };
+        for (int which = 0; which < 2; ++which) {
+            const SplitOperand &s = which ? sp.b : sp.a;
+            const int64_t rows = which || panels == 1 ? s.R : (tiles_m + panels - 1) / panels * 128;
+            sp.part[which] = take((int64_t)s.batch * s.slices * s.R * 4);
+            sp.exps[which] = take((int64_t)s.batch * s.R * 4);
+            sp.dst[which] = take((int64_t)s.batch * rows * ld * 2);
+        }
+        sp.planes = take(g.splits > 1 ? (int64_t)g.splits * p.batch * p.M * p.N * nc * 4 : 0);
+        sp.panels = panels;
+        return off;
+    };
+    int64_t bytes = lay_out(1);
+    for (int panels = 2; bytes > kSplitKeptBytes && panels <= 8 && p.batch == 1 && g.splits == 1 && !p.beta_nz &&
+                         tiles_m / panels * tiles_n >= dev_info().cus; ++panels) {
+        const int64_t b = lay_out(panels);
+        if (b <= kSplitKeptBytes) bytes = b;
+    }
+    if (bytes > kSplitKeptBytes) bytes = lay_out(1);
+    if (bytes > kSplitMaxBytes) return false;
+    sp.cplx = cplx;
+    sp.ws_bytes = std::max<int64_t>(bytes, kSplitFlagBytes + fallback_ws);
+    if (!sizing && d->workspace_bytes < sp.ws_bytes) return false;
+    sp.on = true;
+    return true;
+}
+
 int plan_call(const mb_gemm_desc *d, CallPlan &cp, bool sizing = false) {
+    {
+        CallPlan ps;
+        if (plan_split32(d, ps, sizing)) {
+            cp = ps;
+            return MB_OK;
+        }
+    }
     Peel pe;
     if (plan_peel(d, pe)) {
         cp.n = pe.n;
@@ -1317,6 +1484,7 @@ int plan_call(const mb_gemm_desc *d, CallPlan &cp, bool sizing = false) {
 // the workspace a call plan needs: its copies, then the largest part's own workspace (the
 // parts run one after another)
 int64_t call_ws_bytes(const CallPlan &cp) {
+    if (cp.sp.on) return cp.sp.ws_bytes;
     int64_t ws = 0;
     for (int i = 0; i < cp.n; ++i) ws = std::max<int64_t>(ws, cp.part[i].ws_bytes);
     return cp.copy_bytes + ws;
@@ -1397,10 +1565,21 @@ int cached_plan(const mb_gemm_desc *desc, CallPlan &cp) {
     }
     for (int i = 0; i < cp.n; ++i) each_ptr(cp.part[i], [&](auto *&p) { relocate(p, r); });
     for (int i = 0; i < cp.ncopy; ++i) relocate(cp.copy[i].a.src, r);
+    auto split_ptrs = [](Split32 &s, auto f) { f(s.a.src); f(s.b.src); f(s.g.c); f(s.g.bias); };
+    if (cp.sp.on) split_ptrs(cp.sp, [&](auto *&p) { relocate(p, r); });
     if (hit && cache_mode() == 2) {
         CallPlan fresh;
         const int st = plan_call(desc, fresh);
         bool same = st == MB_OK && fresh.n == cp.n && fresh.ncopy == cp.ncopy && fresh.copy_bytes == cp.copy_bytes;
+        same = same && fresh.sp.on == cp.sp.on && fresh.sp.ws_bytes == cp.sp.ws_bytes &&
+               fresh.sp.g.splits == cp.sp.g.splits && fresh.sp.g.vec_ok == cp.sp.g.vec_ok;
+        if (same && cp.sp.on) {
+            uint64_t px[4], py[4];
+            int nx = 0, ny = 0;
+            split_ptrs(cp.sp, [&](auto *&p) { px[nx++] = (uint64_t)(uintptr_t)p; });
+            split_ptrs(fresh.sp, [&](auto *&p) { py[ny++] = (uint64_t)(uintptr_t)p; });
+            same = memcmp(px, py, sizeof(px)) == 0;
+        }
         for (int i = 0; same && i < cp.ncopy; ++i)
             same = fresh.copy[i].a.src == cp.copy[i].a.src && fresh.copy[i].off == cp.copy[i].off;
         for (int i = 0; same && i < cp.n; ++i) {
@@ -1495,11 +1674,76 @@ void place_copy(T *&ptr, const CallPlan &cp, char *wsb) {
     ptr = (T *)(wsb + cp.copy[k].off + (v - kSentCopy - (uint64_t)k * kSentSpan));
 }
 
+// The split product, then the fp32 plan that runs only if the split raised the flag.
+int run_split32(CallPlan &cp, const mb_gemm_desc *desc, hipStream_t st) {
+    Split32 &sp = cp.sp;
+    if (!desc->workspace || desc->workspace_bytes < sp.ws_bytes) return MB_ERR_WORKSPACE;
+    char *wsb = (char *)desc->workspace;
+    int32_t *flag = (int32_t *)wsb;
+    SplitOperand *ops[2] = {&sp.a, &sp.b};
+    for (int i = 0; i < 2; ++i) {
+        ops[i]->part = (uint32_t *)(wsb + sp.part[i]);
+        ops[i]->exps = (int32_t *)(wsb + sp.exps[i]);
+        ops[i]->dst = wsb + sp.dst[i];
+    }
+    if (launch_split_absmax(sp.a, sp.b, flag, st) != hipSuccess) return MB_ERR_LAUNCH;
+    const int nc = sp.cplx ? 2 : 1, es = 4 * nc;
+    const int rows = sp.panels == 1 ? sp.a.R : (cdiv(sp.a.R, 128) + sp.panels - 1) / sp.panels * 128;
+    GemmArgs g = sp.g;
+    g.a = sp.a.dst;
+    g.b = sp.b.dst;
+    g.ws = wsb + sp.planes;
+    for (int m = 0; m < sp.a.R; m += rows) {
+        SplitOperand a = sp.a, b = sp.b;
+        a.R = std::min(rows, sp.a.R - m);
+        a.src = (const char *)a.src + (int64_t)m * a.rs * es;
+        a.part += m;
+        a.exps += m;
+        if (m > 0) b.R = 0;   // B was split with the first panel
+        if (launch_split32(a, b, flag, st) != hipSuccess) return MB_ERR_LAUNCH;
+        SplitExps x;
+        x.ea = a.exps;
+        x.eb = b.exps;
+        x.ea_bs = a.batch == 1 ? 0 : a.R;
+        x.eb_bs = b.batch == 1 ? 0 : sp.b.R;
+        x.flag = flag;
+        g.M = a.R;
+        g.c = (char *)sp.g.c + (int64_t)m * g.c_rs * es;
+        if (launch_gemm_split32(sp.cplx, g, x, st) != hipSuccess) return MB_ERR_LAUNCH;
+    }
+    if (g.splits > 1) {
+        GemmArgs r = g;
+        r.guard = flag;
+        r.guard_val = 0;
+        if (launch_splitk_reduce(sp.cplx ? C64 : F32, r, st) != hipSuccess) return MB_ERR_LAUNCH;
+    }
+    mb_gemm_desc rest = *desc;
+    rest.workspace = wsb + kSplitFlagBytes;
+    rest.workspace_bytes = desc->workspace_bytes - kSplitFlagBytes;
+    for (int i = 0; i < cp.n; ++i) {
+        Plan &pl = cp.part[i];
+        for (GemmArgs *q : {&pl.gg, &pl.cr}) {
+            q->guard = flag;
+            q->guard_val = 1;
+        }
+        for (PackOp &pk : pl.pack) {
+            pk.a.guard = flag;
+            pk.a.guard_val = 1;
+        }
+        pl.cx.guard = flag;
+        pl.cx.guard_val = 1;
+        const int rs = run_plan(pl, &rest, st, nullptr);
+        if (rs != MB_OK) return rs;
+    }
+    return MB_OK;
+}
+
 int gemm_impl(const mb_gemm_desc *desc, void *stream) {
     CallPlan cp;
     const int st = cache_mode() ? cached_plan(desc, cp) : plan_call(desc, cp);
     if (st != MB_OK) return st;
     if (desc->flags & MB_FLAG_DRY_RUN) return MB_OK;
+    if (cp.sp.on) return run_split32(cp, desc, (hipStream_t)stream);
     if (cp.ncopy > 0) {
         // packed peel: the operand copies first, then the parts on them, each part's own
         // workspace after the copies
@@ -1554,6 +1798,7 @@ int64_t mb_gemm_workspace_bytes(const mb_gemm_desc *desc) {
         return ws;
     }
     CallPlan cp;
+    if (desc && plan_split32(desc, cp, true)) return call_ws_bytes(cp);
     if (desc && plan_packed_peel(desc, cp, true)) return call_ws_bytes(cp);
     Plan pl;
     int st = make_plan(desc, pl);
@@ -1567,10 +1812,11 @@ int mb_plan(const mb_gemm_desc *desc, mb_plan_info *info) {
     Peel pe;
     CallPlan cp;
     // a peeled product reports its core (the strips run on the GEMV / thin kernels)
-    const bool peeled = desc && plan_peel(desc, pe);
-    const bool packed_peel = !peeled && desc && plan_packed_peel(desc, cp, true);
+    const bool split32 = desc && plan_split32(desc, cp, true);
+    const bool peeled = !split32 && desc && plan_peel(desc, pe);
+    const bool packed_peel = !split32 && !peeled && desc && plan_packed_peel(desc, cp, true);
     int st = MB_OK;
-    if (packed_peel)
+    if (packed_peel || split32)
         pl = cp.part[0];
     else
         st = make_plan(peeled ? &pe.part[0] : desc, pl);
@@ -1578,9 +1824,19 @@ int mb_plan(const mb_gemm_desc *desc, mb_plan_info *info) {
     memset(info, 0, sizeof(*info));
     info->family = pl.family;
     info->transposed = pl.p.transposed;
-    info->workspace_bytes = peeled || packed_peel ? mb_gemm_workspace_bytes(desc) : pl.ws_bytes;
+    info->workspace_bytes = split32 || peeled || packed_peel ? mb_gemm_workspace_bytes(desc) : pl.ws_bytes;
     info->split_k = 1;
-    if (pl.family == MB_FAMILY_MFMA) {
+    if (split32) {   // the fp16 product of the split operands (K ping-pong tile, 32 k per stage)
+        const Split32 &sp = cp.sp;
+        const int32_t tile[8] = {128, 128, 32, 2, 4, 4, 1, 1};
+        memcpy(info->tile, tile, sizeof(tile));
+        info->split_k = sp.g.splits;
+        info->swizzle_log = sp.g.swz;
+        info->block = 512;
+        info->grid[0] = cdiv(sp.g.M, 128) * cdiv(sp.g.N, sp.cplx ? 64 : 128);
+        info->grid[1] = sp.g.splits;
+        info->grid[2] = sp.g.batch < 65535 ? sp.g.batch : 65535;
+    } else if (pl.family == MB_FAMILY_MFMA) {
         info->tile[0] = pl.tile.bm;
         info->tile[1] = pl.tile.bn;
         info->tile[2] = 8 * (16 / dtype_size(pl.p.dt));
@@ -1666,7 +1922,9 @@ int mb_tile_candidates(const mb_gemm_desc *desc, int32_t *tiles, int cap) {
         Peel pe;
         CallPlan cp;
         Plan core;
-        if (plan_peel(desc, pe) && make_plan(&pe.part[0], core) == MB_OK) {
+        if (plan_split32(desc, cp, true)) {
+            put(MfmaTile{128, 128, 2, 4, 3}, 0);   // the fp32 tiles, the plan's own among them, are rivals
+        } else if (plan_peel(desc, pe) && make_plan(&pe.part[0], core) == MB_OK) {
             put(core.tile, 0);
         } else if (plan_packed_peel(desc, cp, true)) {
             put(cp.part[0].tile, 0);

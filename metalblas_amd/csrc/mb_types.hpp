@@ -213,6 +213,8 @@ struct GemmArgs {
     int32_t zblocks;     // grid z-blocks when fewer than the batch entries, each workgroup taking
                          // every zblocks-th entry in turn (0: one per entry, at most 65535)
     EpiScalars s;
+    const int32_t *guard;   // set: the kernel runs only where *guard == guard_val (a product queued
+    int32_t guard_val;      // behind a fast path that may have left it the work)
 };
 
 // Final store of one output element: applies the epilogue when enabled.

@@ -210,7 +210,8 @@ template <class T, int ROWS, int NT, bool KC> struct TileLoader {
     }
 };
 
-template <class T, int BM, int BN, int WM, int WN, bool A_KC, bool B_KC>
+// GUARD: the kernel runs only where *g.guard == g.guard_val (fp32, queued behind the fp16 split)
+template <class T, int BM, int BN, int WM, int WN, bool A_KC, bool B_KC, bool GUARD = false>
 __global__ __launch_bounds__(64 * WM * WN) void k_gemm_mfma(GemmArgs g) {
     using P = Pol<T>;
     using Acc = typename P::Acc;
@@ -223,6 +224,8 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_mfma(GemmArgs g) {
     static_assert(TM >= 1 && TN >= 1, "wave tile must hold a 32x32 block");
 
     __shared__ __attribute__((aligned(16))) char smem[2 * STAGE];
+
+    if (GUARD && *g.guard != g.guard_val) return;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave % WM, wn = wave / WM;
@@ -353,18 +356,25 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_mfma(GemmArgs g) {
     }
 }
 
-template <class T, int BM, int BN, int WM, int WN>
-hipError_t launch_tile(bool a_kc, bool b_kc, const GemmArgs &g, dim3 grid, hipStream_t st) {
+template <class T, int BM, int BN, int WM, int WN, bool GUARD>
+hipError_t launch_tile_g(bool a_kc, bool b_kc, const GemmArgs &g, dim3 grid, hipStream_t st) {
     dim3 block(64 * WM * WN);
     if (a_kc && b_kc)
-        hipLaunchKernelGGL((k_gemm_mfma<T, BM, BN, WM, WN, true, true>), grid, block, 0, st, g);
+        hipLaunchKernelGGL((k_gemm_mfma<T, BM, BN, WM, WN, true, true, GUARD>), grid, block, 0, st, g);
     else if (a_kc && !b_kc)
-        hipLaunchKernelGGL((k_gemm_mfma<T, BM, BN, WM, WN, true, false>), grid, block, 0, st, g);
+        hipLaunchKernelGGL((k_gemm_mfma<T, BM, BN, WM, WN, true, false, GUARD>), grid, block, 0, st, g);
     else if (!a_kc && b_kc)
-        hipLaunchKernelGGL((k_gemm_mfma<T, BM, BN, WM, WN, false, true>), grid, block, 0, st, g);
+        hipLaunchKernelGGL((k_gemm_mfma<T, BM, BN, WM, WN, false, true, GUARD>), grid, block, 0, st, g);
     else
-        hipLaunchKernelGGL((k_gemm_mfma<T, BM, BN, WM, WN, false, false>), grid, block, 0, st, g);
+        hipLaunchKernelGGL((k_gemm_mfma<T, BM, BN, WM, WN, false, false, GUARD>), grid, block, 0, st, g);
     return hipGetLastError();
+}
+template <class T, int BM, int BN, int WM, int WN>
+hipError_t launch_tile(bool a_kc, bool b_kc, const GemmArgs &g, dim3 grid, hipStream_t st) {
+    if constexpr (sizeof(T) == 4) {   // fp32
+        if (g.guard) return launch_tile_g<T, BM, BN, WM, WN, true>(a_kc, b_kc, g, grid, st);
+    }
+    return launch_tile_g<T, BM, BN, WM, WN, false>(a_kc, b_kc, g, grid, st);
 }
 
 template <class T>

@@ -30,12 +30,20 @@
 namespace mb {
 namespace m16 {
 
-template <class T, bool A_KC, bool B_KC, bool KTAIL, bool SPLIT> struct Kpp {
+// What the two 32-deep halves of a stage hold.  kPlain: the next 64 k.  kSplitReal / kSplitComplex
+// (K-contiguous fp16, gemm_split32.hip): the high and the low parts of the same 32 k, complex
+// ones as (re, im) pairs along k; the B tile of a complex product is 64 complex columns wide, and
+// the two real columns of each, (re, -im) and (im, re) with the signs of the conjugations, are made
+// from one fragment in registers.
+enum KppMode { kPlain, kSplitReal, kSplitComplex };
+
+template <class T, bool A_KC, bool B_KC, bool KTAIL, KppMode MODE> struct Kpp {
+    static constexpr bool SPLIT = MODE != kPlain, CPLX = MODE == kSplitComplex;
     static constexpr int BM = 128, BN = 128, NW = 8, NB = 4, MS = 16;
     static constexpr int TM = 4, TN = 4;   // 16 x 16 blocks of a 64 x 64 wave tile
     static constexpr int ES = sizeof(T), BK = 128 / ES;
     using TA = Tile16<BM, NW, A_KC, ES, MS>;
-    using TB = Tile16<BN, NW, B_KC, ES, MS>;
+    using TB = Tile16<CPLX ? BN / 2 : BN, NW, B_KC, ES, MS>;
     using Acc = typename AccT<T, MS>::type;
     static constexpr int STAGE = TA::BYTES + TB::BYTES;
     static constexpr int LPW = TA::PER_WAVE + TB::PER_WAVE;   // loads per wave and stage
@@ -45,10 +53,12 @@ template <class T, bool A_KC, bool B_KC, bool KTAIL, bool SPLIT> struct Kpp {
 
     // Sums A[m0.., kbeg..kend) x B[.., n0..) into this wave's half of the tile: on return group 0
     // holds column blocks 0, 1 of its 64 x 64 wave tile in out, group 1 blocks 2, 3.
-    // Ab / Bb: element (m0, kbeg) / (kbeg, n0).
+    // Ab / Bb: element (m0, kbeg) / (kbeg, n0).  Complex: out[0] / out[1] are the real / imaginary
+    // parts of the group's 16 complex columns; sign_re / sign_im: sign bits flipped in the (re, im)
+    // halves of a pair for the real and (after swapping them) the imaginary column.
     __device__ __forceinline__ static void run(const T *Ab, const T *Bb, int64_t lda, int64_t ldb, int rows_a,
                                                int rows_b, int klen, char *smem, int wave, int lane,
-                                               Acc (&out)[2][TM]) {
+                                               Acc (&out)[2][TM], uint32_t sign_re = 0, uint32_t sign_im = 0) {
         const uint32_t smem_lds = lds_addr(smem);
         const int group = wave >> 2, wm = wave & 1, wn = (wave >> 1) & 1;
         const int nk = cdiv(klen, BK), nfull = klen / BK;
@@ -64,7 +74,7 @@ template <class T, bool A_KC, bool B_KC, bool KTAIL, bool SPLIT> struct Kpp {
 #pragma unroll
         for (int j = 0; j < (A_KC ? 1 : TM); ++j) fba[j] = TA::frag_base16(wm * 64, lane, j);
 #pragma unroll
-        for (int j = 0; j < (B_KC ? 1 : TN); ++j) fbb[j] = TB::frag_base16(wn * 64, lane, j);
+        for (int j = 0; j < (B_KC ? 1 : TN); ++j) fbb[j] = TB::frag_base16(wn * (CPLX ? 32 : 64), lane, j);
 
         // load `op` of this wave's share of stage kt (EDGE: the stage that holds the K edge)
         auto load_op = [&](auto edge_tag, int kt, int op) {
@@ -107,9 +117,26 @@ template <class T, bool A_KC, bool B_KC, bool KTAIL, bool SPLIT> struct Kpp {
             for (int s = 0; s < 2; ++s) {
 #pragma unroll
                 for (int j = 0; j < TM; ++j) fa[s][j] = TA::frag16(cur, fba[A_KC ? 0 : j], lane, s, A_KC ? j : 0);
+                if constexpr (CPLX) {
 #pragma unroll
-                for (int i = 0; i < TN; ++i)
-                    fb[s][i] = TB::frag16(cur + TA::BYTES, fbb[B_KC ? 0 : i], lane, s, B_KC ? i : 0);
+                    for (int c = 0; c < TN / 2; ++c) fb[s][2 * c] = TB::frag16(cur + TA::BYTES, fbb[0], lane, s, c);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < TN; ++i)
+                        fb[s][i] = TB::frag16(cur + TA::BYTES, fbb[B_KC ? 0 : i], lane, s, B_KC ? i : 0);
+                }
+            }
+            if constexpr (CPLX) {
+                auto swap = [](uint32_t v) { return __builtin_amdgcn_alignbit(v, v, 16); };
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+#pragma unroll
+                    for (int c = 0; c < TN / 2; ++c) {
+                        const uint4 v = fb[s][2 * c];
+                        fb[s][2 * c + 1] = make_uint4(swap(v.x) ^ sign_im, swap(v.y) ^ sign_im, swap(v.z) ^ sign_im,
+                                                      swap(v.w) ^ sign_im);
+                        fb[s][2 * c] = make_uint4(v.x ^ sign_re, v.y ^ sign_re, v.z ^ sign_re, v.w ^ sign_re);
+                    }
             }
         };
         // The MFMAs of the stage in registers.  Plain: both k halves into one accumulator set.
@@ -448,7 +475,7 @@ template <class T, bool A_KC, bool B_KC, bool KTAIL> struct KppWide {
 
 template <class T, int BM, bool A_KC, bool B_KC, bool KTAIL>
 __global__ __launch_bounds__(512) void k_gemm_kpp(GemmArgs g) {
-    using K = std::conditional_t<BM == 256, KppWide<T, A_KC, B_KC, KTAIL>, Kpp<T, A_KC, B_KC, KTAIL, false>>;
+    using K = std::conditional_t<BM == 256, KppWide<T, A_KC, B_KC, KTAIL>, Kpp<T, A_KC, B_KC, KTAIL, kPlain>>;
     using CS = CStage<T, K::BM, K::BN, K::MS>;
     static_assert(K::XBYTES + CS::BYTES <= K::SMEM, "staged output behind the exchange area");
     __shared__ __attribute__((aligned(1024))) char smem[K::SMEM];
