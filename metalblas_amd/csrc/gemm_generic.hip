@@ -1,9 +1,9 @@
-// Generic LDS-tiled GEMM for every dtype and any element strides, plus the K==0 fill and
+// Generic LDS-tiled GEMM for the float and complex types and any element strides, the K==0 fill and
 // the split-K reduction.
 //
-// This is the register-tiled VALU family: it serves int16/int32/int64 (which have no
-// matrix-core instruction), and any operand the matrix-core loaders cannot stream
-// (unaligned bases, odd leading dimensions, non-unit strides on both axes).  It restates
+// This is the register-tiled VALU family: it serves any operand the matrix-core loaders cannot
+// stream (unaligned bases, odd leading dimensions, non-unit strides on both axes); its integer
+// products run on the 8-bit matrix cores (gemm_limb.hip).  It restates
 // the structure of shaders/int_gemm.h:41-154 (A and B staged through shared memory, a
 // TM x TN micro-tile per thread, accumulate in ACC_T, truncating store) for wave64:
 // BT x BT output tile (BT = 64, 32 or 16), 256 threads as 16x16, (BT/16)^2 accumulators per
@@ -396,8 +396,10 @@ hipError_t launch_generic(int dt, int bt, const GemmArgs &g, hipStream_t st, Lau
     const int tiles = cdiv(g.M, bt) * cdiv(g.N, bt);
     dim3 grid(tiles, g.splits, g.batch < 65535 ? g.batch : 65535), block(256);
     if (shape) *shape = {grid, block};
-    return with_dtype(dt, [&]<class T>() {
-        if (bt == 16) hipLaunchKernelGGL((k_gemm_generic<T, 16>), grid, block, 0, st, g);
+    if (dt == I8 || dt == U8 || dt == I16 || dt == I32 || dt == I64) return launch_limb(dt, bt, g, grid, st);
+    return with_dtype(dt, [&]<class T>() -> hipError_t {
+        if constexpr (Tr<T>::is_int) return hipErrorInvalidValue;   // gemm_limb.hip
+        else if (bt == 16) hipLaunchKernelGGL((k_gemm_generic<T, 16>), grid, block, 0, st, g);
         else if (bt == 32) hipLaunchKernelGGL((k_gemm_generic<T, 32>), grid, block, 0, st, g);
         else hipLaunchKernelGGL((k_gemm_generic<T, 64>), grid, block, 0, st, g);
         return hipGetLastError();

@@ -630,6 +630,9 @@ void plan_generic(const Prob &p, Plan &pl) {
     auto ntiles = [&p](int64_t bt) { return ((p.M + bt - 1) / bt) * ((p.N + bt - 1) / bt) * p.batch; };
     const int64_t tiles = ntiles(64);
     int64_t splits = 1;
+    // K per step: one 8-bit matrix instruction for the integers, one LDS stage for the rest
+    const bool is_int = p.dt != F32 && p.dt != F16 && p.dt != BF16 && p.dt != C64 && p.dt != C32;
+    const int64_t step = is_int ? 64 : 16;
     pl.gen_bt = 64;
     if (p.split_req > 1) {
         splits = p.split_req;
@@ -637,18 +640,24 @@ void plan_generic(const Prob &p, Plan &pl) {
         // few 64 x 64 tiles, short K: 32 x 32 or 16 x 16 tiles fill the CUs with no K slices,
         // so no partial planes and no reduction launch (int32 256^3: 256 tiles of 16 x 16)
         pl.gen_bt = ntiles(32) >= cus ? 32 : 16;
+    } else if (is_int && p.split_req == 0 && tiles < cus && p.K >= 128 && p.K <= 1024) {
+        // 16 x 16 tiles whose four waves share K, however few they are: no planes, one launch
+        // (MI355X, int32, us, K slices of 64 x 64 tiles -> this: 128^3 11.3 -> 3.9, 100 x 300 x 200
+        // 13.7 -> 4.1, 67 x 431 x 153 17.1 -> 4.6; past K = 1024 the slices win)
+        pl.gen_bt = 16;
     } else if (p.split_req == 0 && tiles < cus && p.K >= 128) {
-        // few output tiles: K slices of >= 16 (one LDS step) so that ~2 workgroups run per CU
-        // (int32 256^3: 16 tiles x 16 slices instead of 16 workgroups looping over K)
-        splits = (2LL * cus + tiles - 1) / tiles;
-        const int64_t maxs = p.K / 16;
+        // few output tiles: K slices of whole steps so that ~2 workgroups run per CU, one for the
+        // integers, whose steps are deeper (int32 256 x 256 x 2048 21.1 -> 15.7 us, int64 256 x 256 x
+        // 4096 61 -> 47)
+        splits = ((is_int ? 1LL : 2LL) * cus + tiles - 1) / tiles;
+        const int64_t maxs = p.K / step;
         if (splits > maxs) splits = maxs;
         if (splits > 64) splits = 64;
         if (splits < 1) splits = 1;
     }
     if (splits > 1) {
         int64_t chunk = (p.K + splits - 1) / splits;
-        chunk = (chunk + 15) / 16 * 16;
+        chunk = (chunk + step - 1) / step * step;
         splits = (p.K + chunk - 1) / chunk;
         g.k_chunk = (int)chunk;
         pl.ws_bytes = splits * p.batch * p.M * p.N * acc_size(p.dt);
