@@ -11,15 +11,6 @@
 //     per K slice that the deterministic split-K reduction sums.
 #include "launch.hpp"
 
-// single-vector dot: one row per wave, 8 loads of 16 bytes in flight per lane (tuned on
-// MI355X: 6.5 TB/s on a 16384 x 16384 bf16 matrix with a 2-blocks-per-CU persistent grid)
-#ifndef DOT_R1
-#define DOT_R1 1
-#endif
-#ifndef DOT_U1
-#define DOT_U1 8
-#endif
-
 namespace mb {
 
 namespace {
@@ -561,20 +552,31 @@ template <class T, int NV> hipError_t dot_fast_launch(const GemvArgs &g, hipStre
     if constexpr (NV > 1) {
         if (g.x_row) return dot_xrow_launch<T, NV>(g, st, shape);
     } else {
-        // one vector: workgroup-wide row streams (measured on MI355X, 16384^2 bf16: 77 us,
-        // 6.9 TB/s, against 82 us for a row per wave), 2 rows x 4 loads in flight per thread,
-        // 4 workgroups per CU
-        constexpr int RW = 2, U = 4;
-        int blocks = cdiv(g.rows, RW);
-        const int cap = g.grid_cap > 0 ? 2 * g.grid_cap : 0;
-        if (cap > 0 && blocks > cap) blocks = cap;
+        // One vector.  Rows of more than 256 16-byte chunks: workgroup-wide row streams (MI355X, 16384^2
+        // bf16: 77 us, 6.9 TB/s, against 82 us for a row per wave), 2 rows x 4 loads in flight per
+        // thread, x 2 where a row has fewer than 4 chunks a thread (4 workgroups per CU either way
+        // for long matrices).  Shorter rows, which left a workgroup's threads with one load or none:
+        // a wave streams 2 rows.  MI355X, bf16, cold, us, workgroup streams -> this: 16384 x 1024 12.2
+        // -> 8.6, 4096 x 1024 4.9 -> 4.1, 8192 x 2048 8.9 -> 7.8, 4096^2 8.1 -> 7.8; kept: 2880 x 3288
+        // 6.8 (7.3 a wave), 1024 x 16384 8.1 (11.3).
+        constexpr int RW = 2;
+        const int nch = g.K / Chunk<T>::V;
+        const int cap = 2 * g.grid_cap;   // 4 workgroups per CU
+        int blocks = nch <= 256 ? cdiv(g.rows, 4 * RW) : cdiv(g.rows, RW);
+        const int most = nch < 1024 ? 2 * cap : cap;
+        if (cap > 0 && blocks > most) blocks = most;
         dim3 grid(blocks, 1, g.batch < 65535 ? g.batch : 65535), block(256);
         if (shape) *shape = {grid, block};
-        hipLaunchKernelGGL((k_dot_wg<T, RW, U>), grid, block, 0, st, g);
+        if (nch <= 256)
+            hipLaunchKernelGGL((k_dot_fast<T, 1, RW, 4>), grid, block, 0, st, g);
+        else if (nch < 1024)
+            hipLaunchKernelGGL((k_dot_wg<T, RW, 2>), grid, block, 0, st, g);
+        else
+            hipLaunchKernelGGL((k_dot_wg<T, RW, 4>), grid, block, 0, st, g);
         return hipGetLastError();
     }
-    constexpr int R = NV == 1 ? DOT_R1 : (NV <= 4 ? 4 : (NV == 8 ? 4 : 2));
-    constexpr int U = NV == 1 ? DOT_U1 : (NV <= 4 ? 2 : 1);
+    constexpr int R = NV <= 4 ? 4 : (NV == 8 ? 4 : 2);
+    constexpr int U = NV <= 4 ? 2 : 1;
     const int groups = cdiv(g.rows, R);
     int blocks = cdiv(groups, 4);
     if (g.grid_cap > 0 && blocks > g.grid_cap) blocks = g.grid_cap;
