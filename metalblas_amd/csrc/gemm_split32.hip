@@ -246,13 +246,14 @@ __global__ __launch_bounds__(512) void k_gemm_split32(GemmArgs g, SplitExps x) {
                     else v[r] = ldexpf(out[i][j][r], e);
                 }
                 const bool planes = g.splits > 1;
-                // 4 consecutive outputs as 16-byte stores
-                if (planes ? (g.N & 3) == 0 && gn < g.N : g.vec_ok && !g.epilogue && gn + 3 < g.N) {
+                // 4 consecutive outputs as 16-byte stores (which need only 4-byte alignment)
+                if (gn + 3 < g.N && (planes || (g.c_cs == 1 && !g.epilogue))) {
+                    typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
                     A *dst = planes ? ws + (int64_t)gm * g.N + gn : (A *)(Cb + gm * g.c_rs + gn);
-                    float4 u[sizeof(v) / 16];
+                    f4 u[sizeof(v) / 16];
                     __builtin_memcpy(u, v, sizeof(v));
 #pragma unroll
-                    for (int q = 0; q < (int)sizeof(v) / 16; ++q) ((float4 *)dst)[q] = u[q];
+                    for (int q = 0; q < (int)sizeof(v) / 16; ++q) ((f4 *)dst)[q] = u[q];
                     continue;
                 }
 #pragma unroll

@@ -1411,7 +1411,6 @@ bool plan_split32(const mb_gemm_desc *d, CallPlan &cp, bool sizing) {
     g.a = g.b = nullptr;
     g.a_rs = ld; g.a_cs = 1; g.a_bs = sp.a.d_bs;
     g.b_rs = 1; g.b_cs = ld; g.b_bs = sp.b.d_bs;
-    g.vec_ok = p.c.cs == 1 && p.c.rs % (4 / nc) == 0 && aligned(p.c.ptr, 16) && (p.batch == 1 || p.c.bs % (4 / nc) == 0);
     const int64_t tiles_m = (p.M + 127) / 128, tiles_n = (p.N + bn - 1) / bn, tiles = tiles_m * tiles_n * p.batch;
     if (tiles > kI32Max) return false;
     g.swz = tiles_m >= 8 ? 3 : ilog2_floor(tiles_m);
@@ -1581,7 +1580,7 @@ int cached_plan(const mb_gemm_desc *desc, CallPlan &cp) {
         const int st = plan_call(desc, fresh);
         bool same = st == MB_OK && fresh.n == cp.n && fresh.ncopy == cp.ncopy && fresh.copy_bytes == cp.copy_bytes;
         same = same && fresh.sp.on == cp.sp.on && fresh.sp.ws_bytes == cp.sp.ws_bytes &&
-               fresh.sp.g.splits == cp.sp.g.splits && fresh.sp.g.vec_ok == cp.sp.g.vec_ok;
+               fresh.sp.g.splits == cp.sp.g.splits;
         if (same && cp.sp.on) {
             uint64_t px[4], py[4];
             int nx = 0, ny = 0;
