@@ -138,7 +138,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void k_gemm_limb(GemmArgs g) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int tm, tn, ks, bz0;
-    work_coords(cdiv(g.M, BM), cdiv(g.N, BN), 3, tm, tn, ks, bz0);
+    work_coords(cdiv(g.M, BM), cdiv(g.N, BN), 3, g.xcd_batch, tm, tn, ks, bz0);
     const int wm = KS > 1 ? 0 : wave % WM, wn = KS > 1 ? 0 : wave / WM, wk = KS > 1 ? wave : 0;
     const int m0 = tm * BM + wm * 16 * WT, n0 = tn * BN + wn * 16 * WT;
     const int kbeg = ks * g.k_chunk, kend = min(g.K, kbeg + g.k_chunk);

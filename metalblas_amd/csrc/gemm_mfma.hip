@@ -25,7 +25,7 @@ hipError_t launch_i8_kwhole(const MfmaTile &, bool, bool, const GemmArgs &, dim3
 hipError_t launch_i8_ktail(const MfmaTile &, bool, bool, const GemmArgs &, dim3, hipStream_t);
 hipError_t launch_i8_pp(bool ktail, bool, bool, const GemmArgs &, dim3, hipStream_t);
 hipError_t launch_thin(int dt, bool ktail, const MfmaTile &, bool, bool, const GemmArgs &, dim3, hipStream_t);
-hipError_t launch_deepk(int dt, bool ktail, bool a_kc, bool b_kc, const GemmArgs &g, dim3 grid, hipStream_t st);
+hipError_t launch_ring(int dt, bool ktail, bool a_kc, bool b_kc, const GemmArgs &g, dim3 grid, hipStream_t st);
 }  // namespace m16
 
 namespace {
@@ -47,7 +47,7 @@ constexpr TileEntry kTiles16[] = {
     // K-contiguous, B N-contiguous), k_dotx 4 x 8 (A K-contiguous, up to 16 waves over the
     // whole K)
     {64, 16, 4, 1, 0},   {32, 256, 1, 4, 0},  {32, 128, 1, 4, 0}, {4, 16, 1, 1, 0},  {4, 8, 16, 1, 0},
-    // the deep-K schedule of the 64 x 64 tile (bf16 / fp16): few output tiles, many K slices
+    // the ring schedule of the 64 x 64 tile (bf16 / fp16): few output tiles, with or without K slices
     {64, 64, 2, 2, 2},
     // K ping-pong (mfma_kpp.hpp): two groups of four waves share the K of a 128 x 128 or
     // 256 x 128 tile (bf16 / fp16)
@@ -82,7 +82,7 @@ bool mfma_supported_dtype(int dt) { return dt == BF16 || dt == F16 || dt == F32 
 int mfma_k_align(int dt) { return 16 / dtype_size(dt); }
 
 bool mfma_tile_compiled(int dt, const MfmaTile &t) {
-    if (t.sched >= 2 && dt != BF16 && dt != F16) return false;   // deep-K, K ping-pong: 16-bit floats only
+    if (t.sched >= 2 && dt != BF16 && dt != F16) return false;   // ring, K ping-pong: 16-bit floats only
     if (is16(dt)) return in_table(kTiles16, sizeof(kTiles16) / sizeof(kTiles16[0]), t);
     return in_table(kTiles, sizeof(kTiles) / sizeof(kTiles[0]), t);
 }
@@ -113,10 +113,10 @@ hipError_t launch_mfma(int dt, const MfmaTile &t, bool a_kc, bool b_kc, const Ge
             if ((t.bm == 64 && t.bn == 16) || (t.bm == 32 && (t.bn == 256 || t.bn == 128)) || (t.bm == 4 && t.bn == 16) ||
                 dotx)
                 return m16::launch_thin(dt, !whole, t, a_kc, b_kc, g, grid, st);
-            if (t.sched == 2) {   // deep-K: a 1-D grid of (K slice, tile) workgroups
+            if (t.sched == 2) {   // ring: a 1-D grid of (K slice, tile) workgroups
                 const dim3 g1(tiles * g.splits, 1, grid.z);
                 if (shape) *shape = {g1, dim3(256)};
-                return m16::launch_deepk(dt, !whole, a_kc, b_kc, g, g1, st);
+                return m16::launch_ring(dt, !whole, a_kc, b_kc, g, g1, st);
             }
             if (t.sched == 3) {
                 if (dt == BF16) return m16::launch_bf16_kpp(!whole, t.bm, a_kc, b_kc, g, grid, st);

@@ -202,6 +202,13 @@ void fill_gemm_args(const Prob &p, GemmArgs &g) {
     // cached -> non-temporal): 48 x 2048 x 2048 x 64 (402 MB) 122 -> 103; 16 x 1024^3 (34 MB)
     // 41 -> 48, 96 x 512 x 512 x 64 (50 MB) 19 -> 27.
     g.c_stream = p.batch * p.M * p.N * dtype_size(p.dt) >= (int64_t(256) << 20);
+    // batch entries in XCD-contiguous runs from 16 MiB of operands on (tile_order.hpp); cleared when
+    // K is sliced (run_plan)
+    {
+        const double es = dtype_size(p.dt);
+        const double bytes = es * p.K * ((p.a.bs ? p.batch : 1) * (double)p.M + (p.b.bs ? p.batch : 1) * (double)p.N);
+        g.xcd_batch = p.batch > 1 && bytes >= 16.0 * (1 << 20);
+    }
     g.splits = 1;
     g.k_chunk = (int)(p.K > 0 ? p.K : 1);
     {
@@ -474,11 +481,24 @@ int64_t auto_splits(const Prob &p, int64_t tiles, int bk) {
     return s < 1 ? 1 : s;
 }
 
+// K slices of the 64 x 64 ring: two workgroups per CU from few tiles, slices of at least 1024 (512
+// where the output is so small that its planes cost nothing).  Measured on MI355X (bf16, us by
+// slices): 512 x 1024 x 4096 (128 tiles) 1: 19.9, 2: 17.1, 4: 15.7, 8: 20.3; 17 x 8192 x 2048 (128) 1: 11.1,
+// 2: 10.8, 4: 12.0; 64 x 4096 x 4096 (64) 2: 15.0, 4: 12.7, 8: 15.5; 768 x 768 x 4096 (144) 1: 20.0, 2: 17.6,
+// 4: 22.6; 256 x 256 x 2048 (16) 1: 11.5, 2: 10.7, 4: 8.4, 8: 9.3; 1024 x 1024 x 4096 (256) 1: 20.6, 2: 21.9.
+int64_t ring_splits(const Prob &p, int64_t tiles) {
+    if (p.split_req > 1) return p.split_req;
+    const int cus = dev_info().cus;
+    if (p.split_req != 0 || p.backend != MB_BACKEND_AUTO || p.K < 2048) return 1;
+    const int64_t want = tiles <= cus / 2 ? 2 * cus / tiles : tiles < cus * 3 / 4 ? 2 : 1;
+    return std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(want, p.K / (tiles <= 32 ? 512 : 1024)), 64));
+}
+
 void plan_mfma(const Prob &p, Plan &pl, bool a_kc, bool b_kc, bool thin_ok = false) {
     const int cus = dev_info().cus;
     MfmaTile t;
     bool thin = false;   // the thin-problem tiles below (split for two workgroups per CU)
-    bool deepk = false;  // the deep-K schedule (split for one workgroup per CU)
+    bool deepk = false;  // the ring over a deep K (split for one workgroup per CU)
     // a tile in the descriptor is honoured for the matrix-core backends and for AUTO (where
     // the autotuner puts the tile it measured fastest)
     const bool forced = p.tile[0] > 0 && p.tile[1] > 0;
@@ -501,7 +521,7 @@ void plan_mfma(const Prob &p, Plan &pl, bool a_kc, bool b_kc, bool thin_ok = fal
             {{256, 256, 2, 4, 1}, 1, 1.00}, {{256, 128, 2, 4, 3}, 1, 0.95}, {{256, 256, 2, 2}, 1, 0.85},
             {{256, 128, 2, 2}, 1, 0.66},
             {{128, 256, 2, 2}, 1, 0.66}, {{128, 128, 2, 4, 3}, 1, 0.95}, {{128, 128, 2, 2}, 1, 0.70}, {{128, 64, 2, 2}, 2, 0.65},
-            {{64, 128, 2, 2}, 2, 0.60},  {{64, 64, 2, 2}, 3, 0.40},
+            {{64, 128, 2, 2}, 2, 0.60},  {{64, 64, 2, 2, 2}, 2, 0.40}, {{64, 64, 2, 2}, 3, 0.40},
         };
         const int bk = 128 / dtype_size(p.dt);
         double best = 1e300;
@@ -512,12 +532,25 @@ void plan_mfma(const Prob &p, Plan &pl, bool a_kc, bool b_kc, bool thin_ok = fal
             // the K ping-pong tiles run unsplit unless asked: its waves already share K (1536 x
             // 1536 x 4096, 144 tiles: 33 us, 50 us over 4 slices, 39 us on the best other tile)
             const bool kpp = c.t.sched == 3;
-            const int64_t s = kpp && p.split_req == 0 ? 1 : auto_splits(p, tiles, bk);
+            // The 64 x 64 ring takes the place of the two-buffer 64 x 64 tile below K = 2048 (deeper thin
+            // products run K slices of the tiles below and have the ring as a timed rival), except
+            // for batch entries of a few stages, which run chained on the two-buffer tile.
+            const bool ring = c.t.sched == 2, short_k = p.K <= 4 * bk;
+            const bool f16_mid = dtype_size(p.dt) == 2 && p.K < 2048 && !(p.batch > 1 && short_k);
+            if (ring ? !f16_mid : f16_mid && c.t.bm == 64 && c.t.bn == 64) continue;
+            const int64_t s = kpp && p.split_req == 0 ? 1 : ring ? ring_splits(p, tiles) : auto_splits(p, tiles, bk);
             const int64_t wgs = tiles * s, slots = (int64_t)cus * c.occ;
             const int64_t rounds = (wgs + slots - 1) / slots;
             const int64_t per_cu = std::min<int64_t>(c.occ, (wgs + cus - 1) / cus);
             const int64_t kc = (p.K + s - 1) / s;
             double cost = (double)rounds * per_cu * c.t.bm * c.t.bn * (double)kc / c.eff;
+            // two rings on a CU cover each other's waits (bf16, us: 1024 x 1024 x 4096, one a CU, 20.6;
+            // 512 x 4096 x 4096, two a CU, 29.8)
+            if (ring && per_cu == 2) cost *= 0.8;
+            // a two-buffer 128 x 64 or 64 x 128 tile alone on its CU waits out its loads (bf16, us, against
+            // the 64 x 64 ring: 1408 x 1408 x 1024 12.8, 9.8; 256 x 1024 x 1024 10.3, 7.5), unless they
+            // are a few stages (bmm 8 x 512 x 512 x 256 6.5, K ping-pong 7.5)
+            if (f16_mid && !short_k && c.occ == 2 && per_cu == 1 && !ring) cost *= 1.45;
             // K ping-pong: its ring fills the CU's LDS, so nothing overlaps the start and the end of
             // a tile with the next one's (~4 us a round; 8192 x 1024 x 1024: 24.5 us in two rounds of
             // 128 x 128 against 22.2 in one of 256 x 128; one round of 2048 x 2048 x 4096: 32.7 us
@@ -542,10 +575,9 @@ void plan_mfma(const Prob &p, Plan &pl, bool a_kc, bool b_kc, bool thin_ok = fal
             thin = true;
         }
         // Deep-K products (bf16 / fp16, at most 64 output tiles of 64 x 64, K >= 8192): the
-        // deep-K schedule of the 64 x 64 tile, over K slices of >= 1024 that bring the grid to
-        // about one workgroup per CU.  Measured on MI355X, fp16 128 x 128 x 65536 (64 slices):
-        // 11.4 us for the kernel plus the reduction of its 64 fp32 planes, against 16.2 us for
-        // the rule above (64 x 128 tiles, 64 slices, two LDS buffers).
+        // ring over K slices of >= 1024 that bring the grid to about one workgroup per CU.  Measured on MI355X, fp16 128 x 128 x 65536 (64 slices):
+        // 11.4 us for the kernel plus the reduction of its 64 fp32 planes, against 16.2 us on 64 x 128
+        // tiles (64 slices, two LDS buffers).
         const int64_t t64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch;
         if ((p.dt == MB_DTYPE_BF16 || p.dt == MB_DTYPE_F16) && p.backend == MB_BACKEND_AUTO && p.split_req == 0 &&
             p.K >= 8192 && p.M > 16 && p.N > 16 && t64 <= 64 && std::min<int64_t>(cus / t64, p.K / 1024) >= 2) {
@@ -576,7 +608,7 @@ void plan_mfma(const Prob &p, Plan &pl, bool a_kc, bool b_kc, bool thin_ok = fal
     const int es = dtype_size(p.dt);
     const int BK = 8 * (16 / es);
     const int64_t tiles = ((p.M + t.bm - 1) / t.bm) * ((p.N + t.bn - 1) / t.bn) * p.batch;
-    int64_t splits = t.sched == 3 && p.split_req == 0 ? 1 : auto_splits(p, tiles, BK);
+    int64_t splits = t.sched == 3 && p.split_req == 0 ? 1 : t.sched == 2 ? ring_splits(p, tiles) : auto_splits(p, tiles, BK);
     if (deepk) {
         splits = std::min<int64_t>(cus / tiles, p.K / 1024);
     } else if (thin) {
@@ -1055,6 +1087,7 @@ int run_plan(Plan &pl, const mb_gemm_desc *d, hipStream_t st, LaunchShape *shape
                 g.b = pl.cx.dst;
             }
             g.ws = wsb ? wsb + pl.split_off : nullptr;
+            if (g.splits > 1) g.xcd_batch = 0;
             e = pl.family == MB_FAMILY_MFMA ? launch_mfma(pl.p.dt, pl.tile, pl.a_kc, pl.b_kc, g, st, shape)
                                             : launch_generic(pl.p.dt, pl.gen_bt, g, st, shape);
             if (e != hipSuccess) break;
@@ -1698,6 +1731,7 @@ int run_split32(CallPlan &cp, const mb_gemm_desc *desc, hipStream_t st) {
     const int nc = sp.cplx ? 2 : 1, es = 4 * nc;
     const int rows = sp.panels == 1 ? sp.a.R : (cdiv(sp.a.R, 128) + sp.panels - 1) / sp.panels * 128;
     GemmArgs g = sp.g;
+    if (g.splits > 1) g.xcd_batch = 0;
     g.a = sp.a.dst;
     g.b = sp.b.dst;
     g.ws = wsb + sp.planes;
@@ -1968,8 +2002,7 @@ int mb_tile_candidates(const mb_gemm_desc *desc, int32_t *tiles, int cap) {
                                         {32, 128, 1, 4, 0}, {32, 256, 1, 4, 0}};
         for (const MfmaTile &t : thin) offer(t, 0);
     }
-    // (b) the tile family (matrix-core tiles other than the thin and deep-K schedules), for
-    //     products that are not a single vector.  When the static tile already gives every CU
+    // (b) the tile family (matrix-core tiles other than the thin ones), for products that are not a single vector.  When the static tile already gives every CU
     //     two tiles over a K of at least 1024, tiles of less than a quarter of its area are not
     //     offered: they load more bytes per flop and cannot win there, and timing them (the
     //     32 x 32 register-staged tile takes tens of milliseconds at 8192^3) only delays the
@@ -1982,7 +2015,8 @@ int mb_tile_candidates(const mb_gemm_desc *desc, int32_t *tiles, int cap) {
         const bool plenty = static_tiles >= 2LL * dev_info().cus && p.K >= 1024;
         for (int i = 0; i < n && i < 32; ++i) {
             const MfmaTile &t = list[i];
-            if (thin_tile(t) || t.sched == 2) continue;
+            // (slices of a deep-K plan's ring are offered below)
+            if (thin_tile(t) || (t.sched == 2 && mfma && pl.tile.sched == 2 && p.K >= 8192)) continue;
             if (t.bm > 2 * p.M + 32 || t.bn > 2 * p.N + 32) continue;
             if (plenty && 4LL * t.bm * t.bn < (int64_t)pl.tile.bm * pl.tile.bn) continue;
             offer(t, 0);

@@ -212,6 +212,7 @@ struct GemmArgs {
     int8_t bias_vec;     // bias rows read as 4-element vectors (contiguous, 4-element aligned)
     int8_t c_stream;     // output larger than the last-level cache: non-temporal output stores
     int8_t guard_val;
+    int8_t xcd_batch;    // batch entries in XCD-contiguous runs (tile_order.hpp)
     EpiScalars s;
     const int32_t *guard;   // set: the kernel runs only where *guard == guard_val (a product queued
                             // behind a fast path that may have left it the work)

@@ -675,7 +675,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm16(GemmArgs g) {
     const int wm = wave % WM, wn = wave / WM;
     const int tiles_m = cdiv(g.M, BM), tiles_n = cdiv(g.N, BN);
     int tm, tn, ks, bz0;
-    work_coords(tiles_m, tiles_n, g.swz, tm, tn, ks, bz0);
+    work_coords(tiles_m, tiles_n, g.swz, g.xcd_batch, tm, tn, ks, bz0);
     const int m0 = tm * BM, n0 = tn * BN;
     const int kbeg = ks * g.k_chunk;
     const int kend = min(g.K, kbeg + g.k_chunk);
@@ -928,10 +928,9 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm16(GemmArgs g) {
 // 2 MFMAs per 16-deep k-step per wave; they are not the limit.
 template <int N> __device__ __forceinline__ void vm_wait_n() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
-// Output tile and K slice of workgroup `pid` of a 1-D grid of n = tiles x splits workgroups:
-// workgroup i runs on XCD i % 8, and the workgroups of one XCD take consecutive (slice, tile)
-// indices, so the tiles of a K slice, which read the same slabs of A and B, share one XCD's L2
-// (the remap is a bijection on [0, n) for any n).
+// Output tile and K slice of workgroup `pid` of n = tiles x splits: workgroup i runs on XCD i % 8, and
+// the workgroups of one XCD take consecutive (slice, tile) indices, so the tiles of a K slice, which
+// read the same slabs of A and B, share one XCD's L2 (the remap is a bijection on [0, n) for any n).
 __device__ __forceinline__ void slice_coords(int pid, int n, int tiles, int &tile, int &ks) {
     if (n >= 16) {
         const int xcd = pid & 7, idx = pid >> 3;
@@ -942,10 +941,12 @@ __device__ __forceinline__ void slice_coords(int pid, int n, int tiles, int &til
     ks = pid / tiles;
 }
 
-// XMAP: one workgroup per (tile, K slice) on a 1-D grid in slice_coords order (deep-K products:
-// few output tiles, many K slices); otherwise blockIdx.x is the tile and blockIdx.y the slice.
+// XMAP: one workgroup per (tile, K slice) in slice_coords order (the 64 x 64 ring: products of few
+// output tiles, with or without K slices); otherwise blockIdx.x is the tile and blockIdx.y the slice.
+// STAGED: the output tile leaves through LDS (staged_store_ok holds), for misaligned rows; aligned
+// ones leave from the registers (staging cost the 64 x 64 tile 0.45 us: bf16 512^3 5.1 -> 5.6).
 template <class T, int BM, int BN, int WM, int WN, bool A_KC, bool B_KC, bool KTAIL, int NST, bool XMAP = false,
-          bool NTA = false, bool NTB = false>
+          bool NTA = false, bool NTB = false, bool STAGED = false>
 __global__ __launch_bounds__(64 * WM * WN) void k_thin16(GemmArgs g) {
     constexpr int NW = WM * WN;
     constexpr int WTM = BM / WM, WTN = BN / WN;
@@ -967,14 +968,15 @@ __global__ __launch_bounds__(64 * WM * WN) void k_thin16(GemmArgs g) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave % WM, wn = wave / WM;
     const int tiles_m = cdiv(g.M, BM), tiles_n = cdiv(g.N, BN);
-    int tm, tn, ks, bz0 = blockIdx.z;
+    int tm, tn, ks, bz0;
     if constexpr (XMAP) {
         int tile;
         slice_coords(blockIdx.x, gridDim.x, tiles_m * tiles_n, tile, ks);
+        bz0 = blockIdx.z;
         tm = tile % tiles_m;
         tn = tile / tiles_m;
     } else {
-        work_coords(tiles_m, tiles_n, g.swz, tm, tn, ks, bz0);
+        work_coords(tiles_m, tiles_n, g.swz, g.xcd_batch, tm, tn, ks, bz0);
     }
     const int m0 = tm * BM, n0 = tn * BN;
     const int kbeg = ks * g.k_chunk;
@@ -1056,7 +1058,19 @@ __global__ __launch_bounds__(64 * WM * WN) void k_thin16(GemmArgs g) {
                     for (int j = 0; j < TM; ++j) mma16<T>(acc[i][j], fb[i], fa[j]);
             }
         }
-        store_tile16<T, TM, TN>(g, acc, m0 + wm * WTM, n0 + wn * WTN, bz, ks, lane);
+        if constexpr (STAGED) {
+            using CS = CStage<T, BM, BN, 32>;
+            static_assert(CS::BYTES <= NST * STAGE, "the staged output fits the ring");
+            __syncthreads();   // every wave is done with the ring
+            stage_acc<T, TM, TN, 32, CS>(g, smem, acc, wm * WTM, wn * WTN, m0, n0, bz, lane);
+            __syncthreads();
+            if (g.c_stream)
+                store_staged<T, BM, BN, 32, 64 * NW, true>(g, smem, m0, n0, bz, tid);
+            else
+                store_staged<T, BM, BN, 32, 64 * NW, false>(g, smem, m0, n0, bz, tid);
+        } else {
+            store_tile16<T, TM, TN>(g, acc, m0 + wm * WTM, n0 + wn * WTN, bz, ks, lane);
+        }
         __syncthreads();   // LDS reuse by the next batch iteration
     }
 }
@@ -1076,21 +1090,29 @@ hipError_t launch_thin16(const MfmaTile &t, bool a_kc, bool b_kc, const GemmArgs
     return hipGetLastError();
 }
 
-// The deep-K schedule (sched 2) of the 64 x 64 tile: products with few output tiles and a deep
-// K, split into K slices so that ~256 workgroups stream the operands through a 4-deep ring of
-// 16 KiB LDS-direct stages; the tiles of a slice run on one XCD (slice_coords), so each slab
-// of A and B comes from HBM once.  Measured on MI355X for fp16 128 x 128 x 65536 (64 slices):
-// 7.7 us against 11.6 us for the 2-D grid (tiles of a slice on different XCDs) and 14.4 us
-// for the two-buffer 64 x 128 tile; deeper rings (5..8 stages) measured 8.5-9.4 us.
+// The ring schedule (sched 2) of the 64 x 64 tile: products with few output tiles, over K slices
+// when the tiles leave CUs idle.  A 4-deep ring of 16 KiB LDS-direct stages keeps three stages in
+// flight where the two-buffer tile (k_gemm16) has one, and the load latency is what these products
+// wait for; two workgroups fit a CU.  The tiles of a slice run on one XCD (slice_coords), so each
+// slab of A and B comes from HBM once.  MI355X, us, two-buffer 64 x 64 (or the best 64 x 128 plan) ->
+// ring: bf16 256^3 5.2 -> 4.1, 512^3 6.3 -> 5.1, 1024^3 9.0 -> 7.6, 1024 x 1024 x 2048 18.4 -> 11.4,
+// 1024 x 1024 x 4096 23.2 -> 19.1, 128 x 8192 x 4096 25.2 -> 20.8, 512 x 1024 x 4096 (4 slices) 18.9 ->
+// 15.7; fp16 128 x 128 x 65536 (64 slices) 7.7 against 11.6 for a 2-D grid (tiles of a slice on
+// different XCDs) and 14.4 for the two-buffer 64 x 128 tile; deeper rings (5..8 stages) 8.5-9.4.
+// Rings of 64 x 128 and 128 x 64 tiles (three 24 KiB stages) were slower except at 96 x 4096 x 4096.
 template <class T, bool A_KC, bool B_KC, bool KTAIL>
-hipError_t launch_deepk16_t(const GemmArgs &g, dim3 grid, hipStream_t st) {
-    hipLaunchKernelGGL((k_thin16<T, 64, 64, 2, 2, A_KC, B_KC, KTAIL, 4, true>), grid, dim3(256), 0, st, g);
+hipError_t launch_ring16_t(const GemmArgs &g, dim3 grid, hipStream_t st) {
+    const bool staged = !g.vec_ok && g.c_cs == 1 && g.splits <= 1 && !g.planes;   // staged_store_ok
+    if (staged)
+        hipLaunchKernelGGL((k_thin16<T, 64, 64, 2, 2, A_KC, B_KC, KTAIL, 4, true, false, false, true>), grid, dim3(256), 0, st, g);
+    else
+        hipLaunchKernelGGL((k_thin16<T, 64, 64, 2, 2, A_KC, B_KC, KTAIL, 4, true>), grid, dim3(256), 0, st, g);
     return hipGetLastError();
 }
 template <class T, bool KTAIL>
-hipError_t launch_deepk16(bool a_kc, bool b_kc, const GemmArgs &g, dim3 grid, hipStream_t st) {
-    if (a_kc) return b_kc ? launch_deepk16_t<T, true, true, KTAIL>(g, grid, st) : launch_deepk16_t<T, true, false, KTAIL>(g, grid, st);
-    return b_kc ? launch_deepk16_t<T, false, true, KTAIL>(g, grid, st) : launch_deepk16_t<T, false, false, KTAIL>(g, grid, st);
+hipError_t launch_ring16(bool a_kc, bool b_kc, const GemmArgs &g, dim3 grid, hipStream_t st) {
+    if (a_kc) return b_kc ? launch_ring16_t<T, true, true, KTAIL>(g, grid, st) : launch_ring16_t<T, true, false, KTAIL>(g, grid, st);
+    return b_kc ? launch_ring16_t<T, false, true, KTAIL>(g, grid, st) : launch_ring16_t<T, false, false, KTAIL>(g, grid, st);
 }
 
 // Ping-pong schedule of the 256 x 256 tile with 8 waves, two per SIMD (waves w and w + 4
@@ -1139,7 +1161,7 @@ __global__ __launch_bounds__(512) void k_gemm16pp(GemmArgs g) {
     const int wm = wave % WM, wn = wave / WM;
     const int tiles_m = cdiv(g.M, BM), tiles_n = cdiv(g.N, BN);
     int tm, tn, ks, bz0;
-    work_coords(tiles_m, tiles_n, g.swz, tm, tn, ks, bz0);
+    work_coords(tiles_m, tiles_n, g.swz, g.xcd_batch, tm, tn, ks, bz0);
     const int m0 = tm * BM, n0 = tn * BN;
     const int kbeg = ks * g.k_chunk;
     const int kend = min(g.K, kbeg + g.k_chunk);

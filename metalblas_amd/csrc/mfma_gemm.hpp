@@ -231,7 +231,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_mfma(GemmArgs g) {
     const int wm = wave % WM, wn = wave / WM;
     const int tiles_m = cdiv(g.M, BM), tiles_n = cdiv(g.N, BN);
     int tm, tn, ks, bz0;
-    work_coords(tiles_m, tiles_n, g.swz, tm, tn, ks, bz0);
+    work_coords(tiles_m, tiles_n, g.swz, g.xcd_batch, tm, tn, ks, bz0);
     const int m0 = tm * BM, n0 = tn * BN;
     const int kbeg = ks * g.k_chunk;
     const int kend = min(g.K, kbeg + g.k_chunk);

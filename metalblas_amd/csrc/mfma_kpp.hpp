@@ -483,7 +483,7 @@ __global__ __launch_bounds__(512) void k_gemm_kpp(GemmArgs g) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int tiles_m = cdiv(g.M, K::BM), tiles_n = cdiv(g.N, K::BN);
     int tm, tn, ks, bz0;
-    work_coords(tiles_m, tiles_n, g.swz, tm, tn, ks, bz0);
+    work_coords(tiles_m, tiles_n, g.swz, g.xcd_batch, tm, tn, ks, bz0);
     const int m0 = tm * K::BM, n0 = tn * K::BN;
     const int kbeg = ks * g.k_chunk;
     const int klen = min(g.K, kbeg + g.k_chunk) - kbeg;
