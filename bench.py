@@ -61,10 +61,10 @@ TRAFFIC = {
     "f16_bmm_8x512x512x256": 2.3314e+07,            # k_gemm16 (the tile the tuner took: 128 x 64)
     "f16_bmm_broadcastB": 9.6800e+06,               # k_gemm16 128 x 64
     "f16_splitk_128x128x65536": 3.7852e+07,         # the deep-K k_thin16 64 x 64
-    "c64_gemm_2048_conjA": 3.7610e+08,              # k_gemm_mfma<float> after k_cplx_expand
+    "c64_gemm_2048_conjA": 3.7610e+08,              # measured on k_gemm_mfma<float>; now k_gemm_split32
     "c64_gemv_8192": 5.3758e+08,                    # k_cdot_wg
     "i8_gemm_4096": 1.1798e+08,                     # k_gemm16pp<int8, ...>
-    "i32_gemm_256": 2.9991e+06,                     # k_gemm_generic<int32, 16>
+    "i32_gemm_256": 2.9991e+06,                     # measured on k_gemm_generic; now k_gemm_limb
 }
 
 
